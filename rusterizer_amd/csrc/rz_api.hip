@@ -359,6 +359,7 @@ int build_job(rz_ctx* c, JobPlan& pl) {
         g.msaa_color = ps.msaa_color;
         g.msaa_depth = ps.msaa_depth;
         g.tri_begin = (uint32_t)tri;
+        const uint32_t first_draw = d;
         for (; d < nd && c->draws[d].scene == s; ++d) {
             const PendingDraw& pd = c->draws[d];
             DrawDev& h = dd[d];
@@ -386,6 +387,7 @@ int build_job(rz_ctx* c, JobPlan& pl) {
             if (tri > 0xFFFF0000ull) return fail(c, RZ_ERR_LIMIT, "more than 2^32 triangles in one job");
         }
         g.tri_end = (uint32_t)tri;
+        g.draw = d - first_draw == 1 ? first_draw : MANY_DRAWS;
         tiles += (uint64_t)((ps.W + 15) / 16) * ((ps.H + 15) / 16);
         bins += (uint64_t)g.nbx * g.nby;
         pl.max_nb = std::max(pl.max_nb, g.nbx * g.nby);
@@ -1276,6 +1278,7 @@ extern "C" int rz_render_noalloc(void* stream, uint32_t width, uint32_t height, 
     sc->tri_begin = 0;
     sc->tri_end = ntri_pad;
     sc->out = argb_dev;
+    sc->draw = 0;
     const uint32_t ntiles = ((width + 15) / 16) * ((height + 15) / 16);
     dd->pos = pos_dev;
     dd->col = fragment_shader == RZ_FS_COLOR ? color_dev : nullptr;

@@ -29,6 +29,7 @@ constexpr int SCAN_ITEMS = 8;
 constexpr uint32_t SCAN_TILE = 256 * SCAN_ITEMS;
 constexpr uint32_t NO_TILE = 0xFFFFFFFFu;
 constexpr uint32_t NO_PRIM = 0xFFFFFFFFu;
+constexpr uint32_t MANY_DRAWS = 0xFFFFFFFFu;
 
 // PrimGeom.flags bits: texture coordinates not proven in bounds (see
 // uv_in_bounds); barycentric arguments finite at covered samples (see finite_bary)
@@ -101,7 +102,8 @@ struct SceneCfg {
     uint32_t* out;            // resolved ARGB, W*H words (device)
     uint32_t* msaa_color;     // optional W*H*4 pre-resolve colours
     float* msaa_depth;        // optional W*H*4 pre-resolve depths
-    uint64_t pad2;
+    uint32_t draw;            // the scene's only draw, or MANY_DRAWS
+    uint32_t pad2;
 };
 static_assert(sizeof(SceneCfg) == 80, "SceneCfg layout");
 
@@ -118,18 +120,22 @@ struct SceneRun {
 };
 
 // One rasterizer triangle (RasterizerTriangle, rasterizer/mod.rs:177-184)
-// plus exact-cull helpers, 112 bytes, read with scalar loads by the raster.
+// plus exact-cull helpers, 112 bytes. The leading 80 are what the raster's
+// candidate filter and its matrix path read.
 struct PrimGeom {
     float ax0, ay0, ax1, ay1, ax2, ay2;  // screen points
     float nx0, ny0, nx1, ny1, nx2, ny2;  // edge normals
-    float inv_area;                      // 1 / (2 * area)
-    float z0, z1, z2;                    // screen-space depth
-    uint32_t flags;                      // tie-rule bit per edge (0..2) | PRIM_* bits | fs << 8 | draw << 16
-    float w0, w1, w2;                    // clip-space w
+    float pzx, pzy;                      // depth plane z2 + pzx*(x-ax2) + pzy*(y-ay2)
+    float rscale;                        // |.|: edge scale of the raster's margins (walk_scale; NaN: none); not
+                                         // positive: exact path only
+    float pz0;                           // the depth lower-bound plane's value at point 2 (same slopes)
     uint32_t bbx, bby;                   // clamped pixel bbox: lo | hi << 16
     float zlo;                           // lower bound of every interpolated depth
-    float pz0, pzx, pzy;                 // depth lower-bound plane: pz0 + pzx*(x-bx0) + pzy*(y-by0)
-    uint32_t pad0, pad1;
+    float z2, z0, z1;                    // screen-space depth
+    float inv_area;                      // 1 / (2 * area)
+    uint32_t flags;                      // tie-rule bit per edge (0..2) | PRIM_* bits | fs << 8 | draw << 16
+    float w0, w1, w2;                    // clip-space w
+    uint32_t pad;
 };
 static_assert(sizeof(PrimGeom) == 112, "PrimGeom layout");
 
