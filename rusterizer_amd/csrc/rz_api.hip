@@ -149,8 +149,9 @@ struct rz_ctx {
     uint32_t dcap = 0, scap = 0;
     size_t off_draws = 0, off_mats = 0, off_scenes = 0;
     SceneRun* d_runs = nullptr;
-    SceneRun* h_runs = nullptr;  // pinned
+    uint32_t* h_flags = nullptr;   // pinned: scene flags raised before the raster
     uint32_t* h_sflags = nullptr;  // pinned: scene flags the raster service writes
+    uint32_t* h_oob = nullptr;     // pinned: scenes whose raster read past a texture
     FrameCounters* d_cnt = nullptr;
     FrameCounters* h_cnt = nullptr;  // pinned
 
@@ -298,20 +299,19 @@ int ensure_tables(rz_ctx* c, uint32_t nd, uint32_t ns) {
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     if (c->h_job) (void)hipHostFree(c->h_job);
     if (c->d_job) (void)hipFree(c->d_job);
-    if (c->h_runs) (void)hipHostFree(c->h_runs);
+    if (c->h_flags) (void)hipHostFree(c->h_flags);
     if (c->d_runs) (void)hipFree(c->d_runs);
-    if (c->h_sflags) (void)hipHostFree(c->h_sflags);
     c->h_job = nullptr;
     c->d_job = nullptr;
-    c->h_runs = nullptr;
+    c->h_flags = c->h_sflags = c->h_oob = nullptr;
     c->d_runs = nullptr;
-    c->h_sflags = nullptr;
     c->dcap = c->scap = 0;
     HIP_TRY(c, hipHostMalloc(&c->h_job, bytes, hipHostMallocDefault));
     HIP_TRY(c, hipMalloc(&c->d_job, bytes));
-    HIP_TRY(c, hipHostMalloc(&c->h_runs, sizeof(SceneRun) * scap, hipHostMallocDefault));
+    HIP_TRY(c, hipHostMalloc(&c->h_flags, 3 * sizeof(uint32_t) * scap, hipHostMallocDefault));
+    c->h_sflags = c->h_flags + scap;
+    c->h_oob = c->h_sflags + scap;
     HIP_TRY(c, hipMalloc(&c->d_runs, sizeof(SceneRun) * scap));
-    HIP_TRY(c, hipHostMalloc(&c->h_sflags, sizeof(uint32_t) * scap, hipHostMallocDefault));
     memset(c->h_job, 0, bytes);
     c->job_bytes = bytes;
     c->off_draws = off_d;
@@ -570,6 +570,8 @@ uint64_t ctx_bytes(const rz_ctx* c) {
     return n;
 }
 
+uint32_t init_split(uint32_t draws);
+
 JobBufs job_bufs(const rz_ctx* c) {
     JobBufs b{};
     b.head = reinterpret_cast<const JobHead*>(c->d_job);
@@ -579,6 +581,15 @@ JobBufs job_bufs(const rz_ctx* c) {
     b.runs = c->d_runs;
     b.cnt = c->d_cnt;
     b.svc_flags = c->h_sflags;
+    b.src_head = reinterpret_cast<const JobHead*>(c->h_job);
+    b.src_draws = reinterpret_cast<const DrawDev*>(c->h_job + c->off_draws);
+    b.src_mats = reinterpret_cast<const Mat3*>(c->h_job + c->off_mats);
+    b.src_scenes = reinterpret_cast<const SceneCfg*>(c->h_job + c->off_scenes);
+    b.src_dcap = c->dcap;
+    b.init_split = init_split(c->dcap);
+    b.host_cnt = c->h_cnt;
+    b.host_flags = c->h_flags;
+    b.host_oob = c->h_oob;
     b.cls = c->cls.p;
     b.nsub = c->nsub.p;
     b.suboff = c->suboff.p;
@@ -706,11 +717,16 @@ int svc_prepare(rz_ctx* c, const JobPlan& pl) {
     return svc_ensure(c);
 }
 
+// k_job_init workgroups that share one draw's chunk table: a single draw of
+// millions of triangles has tens of thousands of entries
+uint32_t init_split(uint32_t draws) { return draws <= 32 ? 8u : 1u; }
+
 JobGrid job_grid(const rz_ctx* c, const JobPlan& pl, bool for_graph) {
     JobGrid g{};
-    const uint32_t nd = for_graph ? c->dcap : pl.ndraws;
+    const uint32_t nd = for_graph ? c->dcap : pl.ndraws, ns = for_graph ? c->scap : pl.nscenes;
     const uint32_t nt = for_graph ? (uint32_t)c->cls.cap : pl.ntri;
-    g.draws = (nd + 255) / 256;
+    // a workgroup per draw (or several, init_split), or per 256 words of scene tables
+    g.init = std::min<uint32_t>(std::max(init_split(c->dcap) * nd, (uint32_t)(ns * sizeof(SceneCfg) / 1024)), 1024);
     g.tris = std::min<uint32_t>((nt + 255) / 256, 8192);
     g.clip = (uint32_t)std::min<size_t>(c->clip_tri.cap, 131072);  // slots; k_clip takes CLIP_GROUPS per wave
     const uint64_t chunks = c->geom.cap / CHUNK + (for_graph ? c->scap : pl.nscenes);
@@ -719,7 +735,6 @@ JobGrid job_grid(const rz_ctx* c, const JobPlan& pl, bool for_graph) {
     g.fine = (uint32_t)std::min<uint64_t>(fch, 8192);
     g.raster = c->raster_per_cu ? c->raster_per_cu * (uint32_t)c->n_cu : 0;
     g.ntiles = for_graph ? std::max(c->tiles_cap, pl.ntiles) : pl.ntiles;
-    g.scenes = for_graph ? c->scap : pl.nscenes;
     return g;
 }
 
@@ -729,15 +744,14 @@ int enqueue_eager(rz_ctx* c, const JobPlan& pl) {
     if (rc) return rc;
     SvcState& v = c->pool->svc;
     if (c->prof) HIP_TRY(c, hipEventRecord(c->ev[0], s));
-    HIP_TRY(c, hipMemcpyAsync(c->d_job, c->h_job, c->job_bytes, hipMemcpyHostToDevice, s));
     launch_job(s, job_bufs(c), job_grid(c, pl, false), c->raster_stats, c->prof ? c->ev[1] : nullptr,
                c->prof ? c->ev[2] : nullptr, c->job_svc ? v.ents + c->svc_entry : nullptr, v.host, v.ctl,
                (uint32_t)std::max(c->svc_entry, 0));
     if (c->prof) HIP_TRY(c, hipEventRecord(c->ev[3], s));
     HIP_TRY(c, hipGetLastError());
-    HIP_TRY(c, hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(FrameCounters), hipMemcpyDeviceToHost, s));
-    HIP_TRY(c, hipMemcpyAsync(c->h_runs, c->d_runs, sizeof(SceneRun) * std::max<uint32_t>(pl.nscenes, 1),
-                              hipMemcpyDeviceToHost, s));
+    // the raster's work counts come after the raster reported the rest
+    if (c->raster_stats)
+        HIP_TRY(c, hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(FrameCounters), hipMemcpyDeviceToHost, s));
     HIP_TRY(c, hipEventRecord(c->done, s));
     c->job_graph = false;
     return RZ_OK;
@@ -762,16 +776,11 @@ int enqueue_graph(rz_ctx* c, const JobPlan& pl) {
         }
         hipGraph_t graph = nullptr;
         HIP_TRY(c, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        hipError_t e = hipMemcpyAsync(c->d_job, c->h_job, c->job_bytes, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) {
-            launch_job(s, job_bufs(c), g, c->raster_stats, nullptr, nullptr, svc >= 0 ? v.ents + svc : nullptr,
-                       v.host, v.ctl, (uint32_t)std::max(svc, 0));
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess)
+        launch_job(s, job_bufs(c), g, c->raster_stats, nullptr, nullptr, svc >= 0 ? v.ents + svc : nullptr, v.host,
+                   v.ctl, (uint32_t)std::max(svc, 0));
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess && c->raster_stats)
             e = hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(FrameCounters), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(c->h_runs, c->d_runs, sizeof(SceneRun) * c->scap, hipMemcpyDeviceToHost, s);
         hipError_t e2 = hipStreamEndCapture(s, &graph);
         if (e != hipSuccess || e2 != hipSuccess) {
             if (graph) (void)hipGraphDestroy(graph);
@@ -802,6 +811,7 @@ int enqueue_graph(rz_ctx* c, const JobPlan& pl) {
 int enqueue(rz_ctx* c, bool graph) {
     int rc = ensure_buffers(c, c->plan, Needs{});
     if (rc) return rc;
+    memset(c->h_oob, 0, sizeof(uint32_t) * c->plan.nscenes);
     return graph ? enqueue_graph(c, c->plan) : enqueue_eager(c, c->plan);
 }
 
@@ -848,14 +858,14 @@ int complete_job(rz_ctx* c) {
         // the front end is done and the job posted; the service writes the
         // scenes' final flags to host memory before it marks the job done
         if (!svc_job_done(c)) return 2;
-        for (uint32_t s = 0; s < ns; ++s) c->h_runs[s].flags = __atomic_load_n(&c->h_sflags[s], __ATOMIC_ACQUIRE);
+        for (uint32_t s = 0; s < ns; ++s) c->h_flags[s] = __atomic_load_n(&c->h_sflags[s], __ATOMIC_ACQUIRE);
         c->job_svc = false;
     }
     c->scene_flags.assign(ns, 0);
     uint32_t fl = 0;
     for (uint32_t s = 0; s < ns; ++s) {
-        c->scene_flags[s] = c->h_runs[s].flags;
-        fl |= c->h_runs[s].flags;
+        c->scene_flags[s] = c->h_flags[s] | (c->h_oob[s] ? RZ_FLAG_TEXEL_OOB : 0u);
+        fl |= c->scene_flags[s];
     }
     c->frame_flags = fl;
     c->frame_stats[0] = c->plan.tris;
@@ -1141,6 +1151,11 @@ static_assert(sizeof(JobHead) <= 4 * NA_OFF_DRAW && sizeof(DrawDev) <= 4 * (NA_O
                   4 * NA_OFF_SCENE + sizeof(SceneCfg) <= 4 * NA_TABLE_WORDS && NA_TABLE_WORDS <= WORD_BLOCK,
               "allocation-free job table layout");
 
+struct NoallocResult {
+    FrameCounters cnt;
+    SceneRun run;
+};
+
 // Lays the working buffers of a W x H frame of ntri_pad (padded) triangles
 // out in the scratch array: fixed-size buffers from the frame's shape, then
 // the coarse and fine lists split what is left. Returns false if the fixed
@@ -1154,8 +1169,15 @@ bool noalloc_layout(unsigned char* base, uint32_t ntri_pad, const SceneCfg& sc, 
     b.draws = reinterpret_cast<DrawDev*>(table + NA_OFF_DRAW);
     b.mats = reinterpret_cast<const Mat3*>(table + NA_OFF_MAT);
     b.scenes = reinterpret_cast<const SceneCfg*>(table + NA_OFF_SCENE);
-    b.runs = cv.take<SceneRun>(1);
-    b.cnt = cv.take<FrameCounters>(1);
+    // the counters and the scene's run side by side: one copy reads both back
+    b.cnt = reinterpret_cast<FrameCounters*>(cv.take<NoallocResult>(1));
+    b.runs = reinterpret_cast<SceneRun*>(reinterpret_cast<uintptr_t>(b.cnt) + offsetof(NoallocResult, run));
+    b.src_head = b.head;
+    b.src_draws = b.draws;
+    b.src_mats = b.mats;
+    b.src_scenes = b.scenes;
+    b.src_dcap = 1;
+    b.init_split = 8;
     *maxidx = cv.take<uint32_t>(64);
     const uint64_t nbins = (uint64_t)sc.nbx * sc.nby, T = (uint64_t)(sc.cb >> sc.fts) * (sc.cb >> sc.fts);
     const uint64_t tri_cap = std::max<uint64_t>(ntri_pad, 256);
@@ -1316,35 +1338,32 @@ extern "C" int rz_render_noalloc(void* stream, uint32_t width, uint32_t height, 
     noalloc_layout(base, ntri_pad, *sc, ntiles, b, &d_maxidx, &fixed);
     hipStream_t s = static_cast<hipStream_t>(stream);
 
-    // every index < nv (the reference indexes vertex_buf[idx], render.rs:78-83)
+    // every index < nv (the reference indexes vertex_buf[idx], render.rs:78-83):
+    // k_job_init looks at the largest before any vertex is read
     if (ni) {
-        uint32_t hmax = 0;
         launch_fill_u32(s, d_maxidx, 1, 0u);
         launch_max_index(s, idx_dev, ni, d_maxidx);
-        if (hipMemcpyAsync(&hmax, d_maxidx, sizeof(uint32_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            return noalloc_fail(message, RZ_ERR_HIP, "index check failed");
-        if (hmax >= nv) return noalloc_fail(message, RZ_ERR_ARG, "index out of range");
+        b.max_index = d_maxidx;
+        b.index_limit = nv;
     }
 
     launch_write_words(s, blk, NA_TABLE_WORDS, reinterpret_cast<uint32_t*>(const_cast<JobHead*>(b.head)));
     JobGrid g{};
-    g.draws = 1;
+    g.init = 8;
     g.tris = std::min<uint32_t>((ntri_pad + 255) / 256, 8192);
     g.clip = std::min<uint32_t>(b.clip_cap, 131072);
     g.bins = std::min<uint32_t>(b.prim_cap / CHUNK + 1, 8192);
     g.fine = std::min<uint32_t>(b.pair_cap / CHUNK + b.bins_cap, 8192);
     g.raster = 0;
     g.ntiles = ntiles;
-    g.scenes = 1;
     launch_job(s, b, g, false, nullptr, nullptr);
     if (hipGetLastError() != hipSuccess) return noalloc_fail(message, RZ_ERR_HIP, "kernel launch failed");
-    FrameCounters fc;
-    SceneRun run;
-    if (hipMemcpyAsync(&fc, b.cnt, sizeof(fc), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipMemcpyAsync(&run, b.runs, sizeof(run), hipMemcpyDeviceToHost, s) != hipSuccess ||
+    NoallocResult res;
+    if (hipMemcpyAsync(&res, b.cnt, sizeof(res), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return noalloc_fail(message, RZ_ERR_HIP, "frame failed on the device");
+    const FrameCounters& fc = res.cnt;
+    if (fc.overflow & OVF_INDEX) return noalloc_fail(message, RZ_ERR_ARG, "index out of range");
     if (fc.overflow & OVF_POLY) return noalloc_fail(message, RZ_ERR_LIMIT, "a clipped polygon exceeded 16 vertices");
     // what outgrew the array (rz_resolve_device grows its buffers instead)
     if (fc.overflow & OVF_PRIMS)
@@ -1357,7 +1376,7 @@ extern "C" int rz_render_noalloc(void* stream, uint32_t width, uint32_t height, 
         return noalloc_fail(message, RZ_ERR_LIMIT, "the coarse bin lists do not fit the 128 MiB scratch");
     if (fc.overflow)
         return noalloc_fail(message, RZ_ERR_LIMIT, "the tile bin lists do not fit the 128 MiB scratch");
-    if (flags_out) *flags_out = run.flags;
+    if (flags_out) *flags_out = res.run.flags;
     return RZ_OK;
 }
 
@@ -1414,9 +1433,8 @@ int rz_destroy(rz_ctx* c) {
     release(c->msaa_depth);
     if (c->h_job) (void)hipHostFree(c->h_job);
     if (c->d_job) (void)hipFree(c->d_job);
-    if (c->h_runs) (void)hipHostFree(c->h_runs);
+    if (c->h_flags) (void)hipHostFree(c->h_flags);
     if (c->d_runs) (void)hipFree(c->d_runs);
-    if (c->h_sflags) (void)hipHostFree(c->h_sflags);
     if (c->d_cnt) (void)hipFree(c->d_cnt);
     if (c->h_cnt) (void)hipHostFree(c->h_cnt);
     for (int i = 0; i < 4; ++i)

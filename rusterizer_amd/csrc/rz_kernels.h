@@ -36,7 +36,9 @@ constexpr uint32_t MANY_DRAWS = 0xFFFFFFFFu;
 constexpr uint32_t PRIM_UV_CHECK = 8, PRIM_FINITE_BARY = 16;
 
 // overflow bits: the job must be replayed with larger buffers
-constexpr uint32_t OVF_PRIMS = 1, OVF_CLIP = 2, OVF_PAIRS = 4, OVF_POLY = 8, OVF_FINE = 16, OVF_MATRIX = 32;
+// (OVF_INDEX: not a buffer -- an index is out of range; nothing is rendered)
+constexpr uint32_t OVF_PRIMS = 1, OVF_CLIP = 2, OVF_PAIRS = 4, OVF_POLY = 8, OVF_FINE = 16, OVF_MATRIX = 32,
+                   OVF_INDEX = 64;
 
 struct FrameCounters {
     uint32_t nprims;        // prim slots of the job (each scene starts at a chunk boundary)
@@ -72,7 +74,7 @@ struct JobHead {
 
 // Per-draw state on the device (mesh streams, fragment shader, MVP).
 struct DrawDev {
-    float M[16];             // ((P*V)*W), written by k_job_init
+    float M[16];             // ((P*V)*W), computed by k_job_init
     const float* pos;        // nv*3
     const float* col;        // nv*4 or null
     const float* uv;         // nv*2 or null
@@ -187,20 +189,35 @@ struct JobBufs {
     uint32_t clip_wide;    // clip every polygon with a full wave
     uint32_t exact_paths;  // setup proves nothing: every prim takes the raster's exact paths
     uint32_t* svc_flags;   // raster service: pinned host array of the scenes' final flags
+    // the job tables as the host wrote them (pinned host memory, or the
+    // device tables themselves): k_job_init fills the device tables from them
+    const JobHead* src_head;
+    const DrawDev* src_draws;
+    const Mat3* src_mats;
+    const SceneCfg* src_scenes;
+    uint32_t src_dcap;   // draws the host table has room for
+    uint32_t init_split; // k_job_init workgroups that share a draw's chunks (1 or more)
+    const uint32_t* max_index;  // with max_index: *max_index must be below index_limit (OVF_INDEX)
+    uint32_t index_limit;
+    // results in pinned host memory, written by the raster (null: the host
+    // copies the device's): the counters, and per scene the flags raised
+    // before the raster and whether the raster read past a texture
+    FrameCounters* host_cnt;
+    uint32_t* host_flags;
+    uint32_t* host_oob;
 };
 
 // Grid sizes of one launch sequence. Kernels loop over their work with the
 // device counts, so any grid >= 1 is correct; larger grids only add idle
 // workgroups.
 struct JobGrid {
-    uint32_t draws;      // draw blocks (k_job_init)
+    uint32_t init;       // k_job_init blocks
     uint32_t tris;       // k_classify / k_setup blocks
     uint32_t clip;       // k_clip waves
     uint32_t bins;       // k_bin blocks
     uint32_t fine;       // k_fine_bin blocks
     uint32_t raster;     // persistent raster workgroups; 0 = one one-wave workgroup per quadrant
     uint32_t ntiles;     // tiles the one-per-tile raster grid must cover (>= the job's)
-    uint32_t scenes;     // scene count (k_job_init / k_scene_prep loops)
 };
 
 // A block of words passed to a kernel by value (kernel arguments hold up to

@@ -64,16 +64,6 @@ __device__ __forceinline__ uint32_t hi32(unsigned long long v) { return (uint32_
 // compiler keeps the loads scalar; k_fine_prep calls find_scene_bin per lane.
 // ---------------------------------------------------------------------------
 
-// draw holding padded triangle t: largest d < nd with draws[d].tri_base <= t
-__device__ __forceinline__ uint32_t find_draw(const DrawDev* __restrict__ draws, uint32_t nd, uint32_t t) {
-    uint32_t lo = 0, hi = nd;
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (draws[mid].tri_base <= t) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
 // scene holding global coarse-binning chunk c (scenes without prims share
 // their successor's chunk_base; the largest index is the owner)
 __device__ __forceinline__ uint32_t find_scene_chunk(const SceneRun* __restrict__ runs, uint32_t ns, uint32_t c) {
@@ -117,16 +107,9 @@ __device__ __forceinline__ float4 mat_vec_p(const float* __restrict__ M, float x
     return r;
 }
 
-// per-chunk owner tables, one thread per chunk (the searches run in parallel
-// here instead of serially at the start of every workgroup that needs them):
-// tchunk_map (in k_job_init): the draw of each TRI_ALIGN-triangle chunk (draws
-// start at chunk boundaries); k_pchunk_map: the scene of each CHUNK-prim
-// binning chunk
-__device__ __forceinline__ void tchunk_map(const JobBufs& b) {
-    const uint32_t nc = min((b.head->ntri + TRI_ALIGN - 1) / TRI_ALIGN, b.tchunk_cap), nd = b.head->ndraws;
-    for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x)
-        b.tchunk_draw[c] = find_draw(b.draws, nd, c * TRI_ALIGN);
-}
+// k_pchunk_map: the scene of each CHUNK-prim binning chunk, one thread per
+// chunk (the searches run in parallel here instead of serially at the start of
+// every workgroup that needs them)
 __device__ __forceinline__ void pchunk_map(const JobBufs& b, uint32_t nchunks) {
     const uint32_t nc = min(nchunks, b.pchunk_cap), ns = b.head->nscenes;
     for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x)
@@ -135,29 +118,6 @@ __device__ __forceinline__ void pchunk_map(const JobBufs& b, uint32_t nchunks) {
 __global__ __launch_bounds__(256) void k_pchunk_map(JobBufs b) {
     if (b.cnt->overflow != 0) return;
     pchunk_map(b, b.cnt->nchunks);
-}
-
-// main.rs:147-152: projection * view * world, evaluated left to right
-// (matrix.rs:56-79). One thread per draw; written into the draw descriptor.
-__device__ __forceinline__ void draw_mvp(const JobBufs& b) {
-    const uint32_t nd = b.head->ndraws;
-    for (uint32_t d = blockIdx.x * blockDim.x + threadIdx.x; d < nd; d += gridDim.x * blockDim.x) {
-        const Mat3& m = b.mats[d];
-        float pv[16], out[16];
-        for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j) {
-                float s = 0.0f;
-                for (int k = 0; k < 4; ++k) s = s + m.proj[i * 4 + k] * m.view[k * 4 + j];
-                pv[i * 4 + j] = s;
-            }
-        for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j) {
-                float s = 0.0f;
-                for (int k = 0; k < 4; ++k) s = s + pv[i * 4 + k] * m.world[k * 4 + j];
-                out[i * 4 + j] = s;
-            }
-        for (int i = 0; i < 16; ++i) b.draws[d].M[i] = out[i];
-    }
 }
 
 __device__ __forceinline__ void load_vertex(const DrawDev& dd, uint32_t vi, float4& p, float a[6]) {
@@ -178,37 +138,77 @@ __device__ __forceinline__ void load_vertex(const DrawDev& dd, uint32_t vi, floa
 }
 
 // ---------------------------------------------------------------------------
-// Job start: zero the counters and the per-scene flags (a kernel, not a
-// memset, so the sequence can be captured in a graph).
+// Job start: one launch brings the job tables from the host (read over PCIe,
+// where a copy of its own took 4 us before the first kernel), zeroes the
+// counters and the scenes' flags, and per draw computes its matrix and writes
+// its triangle chunks' entries of the owner table (draws start at chunk
+// boundaries). A workgroup takes a draw (init_split workgroups share one's
+// chunks) and asks for its record, its matrices and the header at once, in one
+// trip to the host; draws past the header's count are in the table's capacity
+// and are not used. Every part is a grid-stride loop, so any grid serves.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void frame_reset(const JobBufs& b) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        FrameCounters* c = b.cnt;
-        c->nprims = 0;
-        c->nprims_raw = 0;
-        c->nclip = 0;
-        c->overflow = 0;
-        c->nchunks = 0;
-        c->mat_len = 0;
-        c->pairs_binned = 0;
-        c->fine_chunks = 0;
-        c->fmat_len = 0;
-        c->fine_total = 0;
-        for (int i = 0; i < 8; ++i) c->q[i] = 0;
-        for (int i = 0; i < 5; ++i) c->rstat[i] = 0;
-    }
-    const uint32_t ns = b.head->nscenes;
-    for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < ns; s += gridDim.x * blockDim.x)
-        b.runs[s].flags = 0;
-}
-
-// k_job_init: the job's three independent first passes in one launch (each a
-// grid-stride loop, so any grid serves): the counter and flag reset, the
-// draws' matrices and the triangle chunks' draws
 __global__ __launch_bounds__(256) void k_job_init(JobBufs b) {
-    frame_reset(b);
-    draw_mvp(b);
-    tchunk_map(b);
+    __shared__ uint32_t draw[sizeof(DrawDev) / 4u], head[sizeof(JobHead) / 4u];
+    __shared__ float mats[48], pv[16];
+    constexpr uint32_t HW = sizeof(JobHead) / 4u, DW = sizeof(DrawDev) / 4u, SW = sizeof(SceneCfg) / 4u;
+    const uint32_t t = threadIdx.x, split = b.init_split;
+    const uint32_t* src_scenes = reinterpret_cast<const uint32_t*>(b.src_scenes);
+    const uint32_t stride = gridDim.x * 256u, first = blockIdx.x * 256u + t;
+    uint32_t hw = 0, dw = 0;
+    float mw = 0.0f;
+    auto fetch = [&](uint32_t u) {
+        const uint32_t d = u / split;
+        if (d < b.src_dcap) {
+            if (t < DW) dw = reinterpret_cast<const uint32_t*>(b.src_draws + d)[t];
+            if (t < 48) mw = reinterpret_cast<const float*>(b.src_mats + d)[t];
+        }
+    };
+    if (t < HW) hw = reinterpret_cast<const uint32_t*>(b.src_head)[t];
+    fetch(blockIdx.x);
+    if (t < HW) head[t] = hw;
+    if (blockIdx.x == 0) {
+        uint32_t* cnt = reinterpret_cast<uint32_t*>(b.cnt);
+        if (t < sizeof(FrameCounters) / 4u) cnt[t] = 0u;
+        if (t < HW) reinterpret_cast<uint32_t*>(const_cast<JobHead*>(b.head))[t] = hw;
+    }
+    __syncthreads();
+    const uint32_t nd = reinterpret_cast<const JobHead*>(head)->ndraws, ns = reinterpret_cast<const JobHead*>(head)->nscenes;
+    if (first == 0 && b.max_index && *b.max_index >= b.index_limit) b.cnt->overflow = OVF_INDEX;
+    for (uint32_t i = first; i < ns * SW; i += stride)
+        reinterpret_cast<uint32_t*>(const_cast<SceneCfg*>(b.scenes))[i] = src_scenes[i];
+    for (uint32_t s = first; s < ns; s += stride) b.runs[s].flags = 0;
+    for (uint32_t u = blockIdx.x; u < nd * split; u += gridDim.x) {
+        const uint32_t d = u / split, part = u % split;
+        if (u != blockIdx.x) fetch(u);
+        if (t < DW) draw[t] = dw;
+        if (t < 48) mats[t] = mw;
+        __syncthreads();
+        const DrawDev& src = *reinterpret_cast<const DrawDev*>(draw);
+        const uint32_t c0 = src.tri_base / TRI_ALIGN;
+        const uint32_t nc = min((src.ntri + TRI_ALIGN - 1u) / TRI_ALIGN, b.tchunk_cap - min(c0, b.tchunk_cap));
+        for (uint32_t c = part * 256u + t; c < nc; c += split * 256u) b.tchunk_draw[c0 + c] = d;
+        // main.rs:147-152: projection * view * world, evaluated left to right
+        // (matrix.rs:56-79), a thread an element
+        const float *world = mats, *view = mats + 16, *proj = mats + 32;
+        const uint32_t i = (t & 15u) / 4u, j = t & 3u;
+        if (t < 16) {
+            float s = 0.0f;
+            for (int k = 0; k < 4; ++k) s = s + proj[i * 4 + k] * view[k * 4 + j];
+            pv[t] = s;
+        }
+        __syncthreads();
+        if (part == 0) {
+            uint32_t* dst = reinterpret_cast<uint32_t*>(b.draws + d);
+            if (t < 16) {
+                float s = 0.0f;
+                for (int k = 0; k < 4; ++k) s = s + pv[i * 4 + k] * world[k * 4 + j];
+                dst[t] = __float_as_uint(s);
+            } else if (t < DW) {
+                dst[t] = dw;
+            }
+        }
+        __syncthreads();  // the LDS copies are the next draw's
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -222,6 +222,7 @@ __global__ __launch_bounds__(256) void k_job_init(JobBufs b) {
 __global__ __launch_bounds__(256) void k_classify(JobBufs b, const uint32_t* __restrict__ tchunk_draw,
                                                   const DrawDev* __restrict__ draws) {
     __shared__ uint32_t wcount[4], wbase[4];
+    if (uniform(b.cnt->overflow) & OVF_INDEX) return;  // no vertex is read through a bad index
     const uint32_t NT = b.head->ntri;
     const uint32_t wave = threadIdx.x >> 6;
     uint32_t wneed = 0;  // the wave's clipped triangles over all its chunks
@@ -888,6 +889,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const float* __restrict__ clip_out) {
     __shared__ PrimGeom stage[SETUP_STAGE];
     __shared__ uint32_t poff[256], pcls[256];  // per triangle of the chunk: first prim (chunk-relative), class
+    if (uniform(b.cnt->overflow) != 0) return;
     const uint32_t NT = b.head->ntri;
     const uint32_t prim_cap = b.prim_cap;
     // the chunk table words of the workgroup's next chunk are loaded one
@@ -1834,7 +1836,7 @@ __device__ __forceinline__ float exact_depth(const PrimGeom& g, float sx, float 
 // share the shading tasks; R = 1: the workgroup is one wave and takes
 // quadrant quad of the tile alone.
 template <bool STATS, uint32_t R>
-__device__ __forceinline__ void raster_tile(SceneRun* runs, const RasterIn& in, uint32_t slot, uint32_t quad, uint4 tr1,
+__device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, const RasterIn& in, uint32_t slot, uint32_t quad, uint4 tr1,
                                             float* lut, ShadeLds<R>& sh,
                                             uint32_t& st_entries, uint32_t& st_cand, uint32_t& st_hits,
                                             uint32_t& st_cov, uint32_t& st_shaded) {
@@ -2275,7 +2277,10 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, const RasterIn& in, 
     const uint32_t cb1 = (vmask & 2u) ? wargb[(slots >> 8) & 0xFFu] : CLEAR_COLOR;
     const uint32_t cb2 = (vmask & 4u) ? wargb[(slots >> 16) & 0xFFu] : CLEAR_COLOR;
     const uint32_t cb3 = (vmask & 8u) ? wargb[slots >> 24] : CLEAR_COLOR;
-    if (ballot(oob) && lane == 0) atomicOr(&runs[s].flags, RZ_FLAG_TEXEL_OOB);
+    if (ballot(oob) && lane == 0) {
+        atomicOr(&runs[s].flags, RZ_FLAG_TEXEL_OOB);
+        if (host_oob) host_oob[s] = 1u;
+    }
     uint32_t l3 = lane;
     asm volatile("" : "+v"(l3));
     const uint32_t px3 = qx0 + (l3 & 7), py3 = qy0 + (l3 >> 3);
@@ -2291,6 +2296,19 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, const RasterIn& in, 
             *reinterpret_cast<uint4*>(sc.msaa_color + o * 4) = c4;
         }
     }
+}
+
+// What the host reads after the job, written to its pinned memory by one
+// workgroup of the raster (every counter is final before it, and a copy after
+// the job takes 4 us each): the counters, and the scenes' flags so far. The
+// raster's own flag goes to host_oob.
+__device__ __forceinline__ void report_job(const JobBufs& b) {
+    if (!b.host_cnt) return;
+    constexpr uint32_t CW = sizeof(FrameCounters) / 4u;
+    for (uint32_t i = threadIdx.x; i < CW; i += blockDim.x)
+        reinterpret_cast<uint32_t*>(b.host_cnt)[i] = reinterpret_cast<const uint32_t*>(b.cnt)[i];
+    const uint32_t ns = b.head->nscenes;
+    for (uint32_t s = threadIdx.x; s < ns; s += blockDim.x) b.host_flags[s] = b.runs[s].flags;
 }
 
 // Persistent raster (raster_per_cu > 0): raster_per_cu workgroups of four
@@ -2310,6 +2328,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
     __shared__ ShadeLds<4> sh;
     lut[threadIdx.x] = kByteToFloat.v[threadIdx.x];
     __syncthreads();
+    if (blockIdx.x == 0) report_job(b);
     if (uniform(b.cnt->overflow) != 0) return;
     uint32_t st_entries = 0, st_cand = 0, st_hits = 0, st_cov = 0, st_shaded = 0;
     const uint32_t nt = b.head->ntiles;
@@ -2330,7 +2349,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
         const uint32_t tile = next_tile;
         __syncthreads();
         if (tile == NO_TILE) break;
-        raster_tile<STATS, 4>(b.runs, in, tile, 0u, uint4{}, lut, sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
+        raster_tile<STATS, 4>(b.runs, b.host_oob, in, tile, 0u, uint4{}, lut, sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
     }
     if (STATS) {  // the last two counts are per lane
         for (int o = 32; o >= 1; o >>= 1) {
@@ -2388,10 +2407,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 
     // asked for together with the counters that say whether it holds anything
     const uint4 tr = tile_rec[min(qs, 4u * b.tile_cap - 1u)];
     const uint32_t nq = 4u * b.head->ntiles;
+    if (blockIdx.x == 0) report_job(b);
     if (uniform(b.cnt->overflow) != 0) return;
     uint32_t st_entries = 0, st_cand = 0, st_hits = 0, st_cov = 0, st_shaded = 0;
     if (qs < nq)
-        raster_tile<STATS, 1>(b.runs, in, qs >> 2, qs & 3u, tr, sh.lut(), sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
+        raster_tile<STATS, 1>(b.runs, b.host_oob, in, qs >> 2, qs & 3u, tr, sh.lut(), sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
     if (STATS) {  // every workgroup writes its counts, zeros past the last quadrant
         for (int o = 32; o >= 1; o >>= 1) {  // the last two counts are per lane
             st_cov += __shfl_xor(st_cov, o);
@@ -2485,6 +2505,7 @@ static uint32_t at_least1(uint32_t v) { return v ? v : 1u; }
 // visible. A job without tiles is finished at once.
 // ---------------------------------------------------------------------------
 __global__ void k_svc_post(JobBufs b, SvcEntry* e, SvcHost* host, SvcCtl* ctl, uint32_t index) {
+    report_job(b);
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (b.cnt->overflow != 0) return;
     const uint32_t nt = b.head->ntiles;
@@ -2714,7 +2735,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                           svc_ptr<uint2>(&j->flist),   svc_ptr<uint4>(&j->tile_rec), svc_ptr<SceneCfg>(&j->scenes),
                           svc_ptr<DrawDev>(&j->draws)};
         SceneRun* runs = svc_ptr_mut<SceneRun>(&j->runs);
-        raster_tile<false, 4>(runs, in, t, 0u, uint4{}, lut, sh, st0, st1, st2, st3, st4);
+        raster_tile<false, 4>(runs, nullptr, in, t, 0u, uint4{}, lut, sh, st0, st1, st2, st3, st4);
         pend_e = e;
         pend_g = g;
         pend_nt = nt;
@@ -2729,9 +2750,7 @@ void launch_raster_service(hipStream_t s, uint32_t grid, SvcEntry* ents, uint32_
 
 void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_stats, hipEvent_t ev_bin,
                 hipEvent_t ev_raster, SvcEntry* svc, SvcHost* svc_host, SvcCtl* svc_ctl, uint32_t svc_index) {
-    const uint32_t scene_blocks = (g.scenes + 255) / 256;
-    const uint32_t tchunk_blocks = std::min<uint32_t>((g.tris + 255) / 256 + 1, 1024u);
-    k_job_init<<<at_least1(std::max({scene_blocks, g.draws, tchunk_blocks})), 256, 0, s>>>(b);
+    k_job_init<<<at_least1(g.init), 256, 0, s>>>(b);
     k_classify<<<at_least1(std::min<uint32_t>(g.tris, 2048u)), 256, 0, s>>>(b, b.tchunk_draw, b.draws);
     k_clip<<<at_least1((g.clip + CLIP_GROUPS - 1) / CLIP_GROUPS), 64, 0, s>>>(b);
     if (b.tri_cap <= SCAN_ONE_MAX) {
