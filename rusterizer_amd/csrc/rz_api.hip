@@ -156,7 +156,7 @@ struct rz_ctx {
     FrameCounters* h_cnt = nullptr;  // pinned
 
     // pipeline buffers
-    DBuf<uint32_t> cls, nsub, suboff, parts;
+    DBuf<uint32_t> cls, nsub, wave_prims, chunk_off, parts;
     DBuf<unsigned long long> parts64;
     DBuf<uint32_t> clip_tri, clip_draw;
     DBuf<float> clip_out;  // MAXV * 10 floats per slot
@@ -468,7 +468,8 @@ int size_buffers(rz_ctx* c, const JobPlan& pl, const Needs& n_in, G& g) {
         return fail(c, RZ_ERR_LIMIT, "job needs more than 2^32 pipeline entries");
     const size_t cls = g(c->cls, std::max<uint64_t>(NT, 256));
     g(c->nsub, cls);
-    g(c->suboff, cls);
+    g(c->wave_prims, cls / 64 + 4);
+    g(c->chunk_off, cls / TRI_ALIGN + 1);
     const size_t geom = g(c->geom, n.prims);
     g(c->attrs, geom * ATTR_STRIDE);
     g(c->uvat, geom * UV_STRIDE);
@@ -557,7 +558,7 @@ uint64_t held(const DBuf<T>& b) {
 
 // device bytes of the context's pipeline buffers, outputs and tables
 uint64_t ctx_bytes(const rz_ctx* c) {
-    uint64_t n = held(c->cls) + held(c->nsub) + held(c->suboff) + held(c->parts) + held(c->parts64) +
+    uint64_t n = held(c->cls) + held(c->nsub) + held(c->wave_prims) + held(c->chunk_off) + held(c->parts) + held(c->parts64) +
                  held(c->clip_tri) + held(c->clip_draw) + held(c->clip_out) + held(c->geom) +
                  held(c->attrs) + held(c->uvat) + held(c->pbin) + held(c->bin_counts) + held(c->bin_offsets) + held(c->list) +
                  held(c->bin_rng) + held(c->tile_rec) + held(c->fchunk_rec) + held(c->tchunk_draw) +
@@ -592,7 +593,8 @@ JobBufs job_bufs(const rz_ctx* c) {
     b.host_oob = c->h_oob;
     b.cls = c->cls.p;
     b.nsub = c->nsub.p;
-    b.suboff = c->suboff.p;
+    b.wave_prims = c->wave_prims.p;
+    b.chunk_off = c->chunk_off.p;
     b.clip_tri = c->clip_tri.p;
     b.clip_draw = c->clip_draw.p;
     b.clip_out = c->clip_out.p;
@@ -1186,7 +1188,10 @@ bool noalloc_layout(unsigned char* base, uint32_t ntri_pad, const SceneCfg& sc, 
     const uint64_t mat = nbins * (prims / CHUNK + 1);
     b.cls = cv.take<uint32_t>(tri_cap);
     b.nsub = cv.take<uint32_t>(tri_cap);
-    b.suboff = cv.take<uint32_t>(tri_cap);
+    // (one word a triangle held these offsets once: the room it leaves is kept
+    // unused, so that the lists hold what they held)
+    b.wave_prims = cv.take<uint32_t>(tri_cap);
+    b.chunk_off = b.wave_prims + tri_cap / 64;
     b.tchunk_draw = cv.take<uint32_t>(tri_cap / TRI_ALIGN + 1);
     b.geom = cv.take<PrimGeom>(prims);
     b.attrs = cv.take<float>(prims * ATTR_STRIDE);
@@ -1404,7 +1409,8 @@ int rz_destroy(rz_ctx* c) {
     if (c->graph) (void)hipGraphExecDestroy(c->graph);
     release(c->cls);
     release(c->nsub);
-    release(c->suboff);
+    release(c->wave_prims);
+    release(c->chunk_off);
     release(c->parts);
     release(c->parts64);
     release(c->clip_tri);
@@ -1623,7 +1629,8 @@ int rz_trim(rz_ctx* c) {
     }
     release(c->cls);
     release(c->nsub);
-    release(c->suboff);
+    release(c->wave_prims);
+    release(c->chunk_off);
     release(c->parts);
     release(c->parts64);
     release(c->clip_tri);

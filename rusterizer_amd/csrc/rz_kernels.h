@@ -154,8 +154,9 @@ struct JobBufs {
     FrameCounters* cnt;
     // geometry
     uint32_t* cls;
-    uint32_t* nsub;
-    uint32_t* suboff;
+    uint32_t* nsub;       // rasterizer triangles of each clipped triangle
+    uint32_t* wave_prims; // rasterizer triangles of each 64 triangles
+    uint32_t* chunk_off;  // per TRI_ALIGN-triangle chunk: the rasterizer triangles of all earlier ones
     uint32_t* clip_tri;   // clipped triangle of each clip slot
     uint32_t* clip_draw;  // its draw
     float* clip_out;

@@ -6,7 +6,7 @@
 // same association, Rust's saturating float->int casts).
 //
 // Pipeline of one job (S scenes, D draws; all on one stream):
-//   k_job_init (counter reset, MVPs) -> k_classify -> k_clip -> scan(nsub)
+//   k_job_init (tables, counter reset, MVPs) -> k_classify -> k_clip
 //   -> k_scene_prep -> k_setup                                  (geometry)
 //   -> k_bin<count> -> scan -> k_bin<scatter>                   (coarse bins)
 //   -> k_fine_prep -> scan64 -> k_fine_bin<count> -> scan
@@ -64,17 +64,6 @@ __device__ __forceinline__ uint32_t hi32(unsigned long long v) { return (uint32_
 // compiler keeps the loads scalar; k_fine_prep calls find_scene_bin per lane.
 // ---------------------------------------------------------------------------
 
-// scene holding global coarse-binning chunk c (scenes without prims share
-// their successor's chunk_base; the largest index is the owner)
-__device__ __forceinline__ uint32_t find_scene_chunk(const SceneRun* __restrict__ runs, uint32_t ns, uint32_t c) {
-    uint32_t lo = 0, hi = ns;
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (runs[mid].chunk_base <= c) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
 __device__ __forceinline__ uint32_t find_scene_tile(const SceneCfg* __restrict__ sc, uint32_t ns, uint32_t t) {
     uint32_t lo = 0, hi = ns;
     while (hi - lo > 1) {
@@ -105,19 +94,6 @@ __device__ __forceinline__ float4 mat_vec_p(const float* __restrict__ M, float x
     r.z = (((0.0f + M[8] * x) + M[9] * y) + M[10] * z) + M[11] * 1.0f;
     r.w = (((0.0f + M[12] * x) + M[13] * y) + M[14] * z) + M[15] * 1.0f;
     return r;
-}
-
-// k_pchunk_map: the scene of each CHUNK-prim binning chunk, one thread per
-// chunk (the searches run in parallel here instead of serially at the start of
-// every workgroup that needs them)
-__device__ __forceinline__ void pchunk_map(const JobBufs& b, uint32_t nchunks) {
-    const uint32_t nc = min(nchunks, b.pchunk_cap), ns = b.head->nscenes;
-    for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x)
-        b.pchunk_scene[c] = find_scene_chunk(b.runs, ns, c);
-}
-__global__ __launch_bounds__(256) void k_pchunk_map(JobBufs b) {
-    if (b.cnt->overflow != 0) return;
-    pchunk_map(b, b.cnt->nchunks);
 }
 
 __device__ __forceinline__ void load_vertex(const DrawDev& dd, uint32_t vi, float4& p, float a[6]) {
@@ -266,11 +242,10 @@ __global__ __launch_bounds__(256) void k_classify(JobBufs b, const uint32_t* __r
         // pass 1 marks clipped triangles with 2; their slots come below
         const bool need = live && c == 2;
         wneed += (uint32_t)__popcll(__ballot(need));
-        if (t < NT) {
-            b.cls[t] = need ? 2u : c;
-            b.nsub[t] = need ? 0u : c;  // Inside -> 1 rasterizer triangle, Outside / padding -> 0;
-                                        // clipped: written by k_clip
-        }
+        if (t < NT) b.cls[t] = need ? 2u : c;
+        // Inside -> 1 rasterizer triangle; k_clip adds the clipped ones'
+        const uint32_t inside = (uint32_t)__popcll(ballot(c == 1u));
+        if (lane_id() == 0) b.wave_prims[blk * 4u + wave] = inside;
     }
     // one clip-list reservation per workgroup for all its chunks (a global
     // atomic per chunk would serialize thousands of workgroups on one counter)
@@ -437,7 +412,10 @@ __device__ __forceinline__ bool clip_polygon(const JobBufs& b, uint32_t slot, bo
     } else if (n > 0) {
         if (gl == 0) atomicOr(&b.runs[scene].flags, RZ_FLAG_CLIP_FEWER);
     }
-    if (gl == 0) b.nsub[t] = ntris;
+    if (gl == 0) {
+        b.nsub[t] = ntris;
+        if (ntris != 0) atomicAdd(&b.wave_prims[t / 64u], ntris);
+    }
     return false;
 }
 
@@ -611,13 +589,16 @@ void launch_scan(hipStream_t s, const T* in, T* out, uint32_t n_host, const uint
 }
 
 // ---------------------------------------------------------------------------
-// k_scene_prep: one workgroup. From the scanned fan counts, each scene's
-// rasterizer triangle range, its CHUNK-aligned prim slots, its binning
-// chunks and the base of its coarse count matrix (bins x chunks).
+// k_scene_prep: one workgroup. Scans the chunks' rasterizer triangles (k_setup
+// scans inside a chunk), then each scene's rasterizer triangle range, its
+// CHUNK-aligned prim slots, its binning chunks and the base of its coarse count
+// matrix (bins x chunks). Scanning chunks instead of triangles keeps it one
+// launch at any size (10M triangles: 41k chunks, 10 passes, 42 us) where a scan of
+// all triangles took three more launches (59 us there; of a 15k-triangle scene 19
+// us against 5 now) and 16 bytes of traffic per triangle.
 // ---------------------------------------------------------------------------
-// (blockDim.x threads; total = the job's rasterizer triangles; returns the
-// job's binning chunks and coarse matrix length in every thread)
-__device__ __forceinline__ uint2 scene_prep(const JobBufs& b, uint32_t total, uint32_t* l1, uint32_t* l2) {
+// (blockDim.x threads; total = the job's rasterizer triangles)
+__device__ __forceinline__ void scene_prep(const JobBufs& b, uint32_t total, uint32_t* l1, uint32_t* l2) {
     const uint32_t ns = b.head->nscenes, NT = b.head->ntri;
     uint32_t run_ch = 0, run_mat = 0;
     for (uint32_t off = 0; off < ns; off += blockDim.x) {
@@ -625,8 +606,8 @@ __device__ __forceinline__ uint2 scene_prep(const JobBufs& b, uint32_t total, ui
         uint32_t nch = 0, nmat = 0, beg = 0, np = 0;
         if (s < ns) {
             const SceneCfg& sc = b.scenes[s];
-            beg = sc.tri_begin < NT ? b.suboff[sc.tri_begin] : total;
-            const uint32_t end = sc.tri_end < NT ? b.suboff[sc.tri_end] : total;
+            beg = sc.tri_begin < NT ? b.chunk_off[sc.tri_begin / TRI_ALIGN] : total;
+            const uint32_t end = sc.tri_end < NT ? b.chunk_off[sc.tri_end / TRI_ALIGN] : total;
             np = end - beg;
             nch = (np + CHUNK - 1) / CHUNK;
             nmat = sc.nbx * sc.nby * nch;
@@ -656,34 +637,42 @@ __device__ __forceinline__ uint2 scene_prep(const JobBufs& b, uint32_t total, ui
         if (run_mat > b.mat_cap) o |= OVF_MATRIX;
         if (o) atomicOr(&c->overflow, o);
     }
-    return make_uint2(run_ch, run_mat);
 }
 __global__ __launch_bounds__(1024) void k_scene_prep(JobBufs b) {
     __shared__ uint32_t l1[16], l2[16];
-    (void)scene_prep(b, b.cnt->nprims_raw, l1, l2);
-}
-
-// The scan of the prims per triangle, k_scene_prep and k_pchunk_map by one
-// workgroup, for jobs of at most SCAN_ONE_MAX (padded) triangles: one launch
-// instead of three. The totals each step needs pass in registers (every
-// thread holds them); the barriers order each step's global writes before
-// the next step's reads.
-__global__ __launch_bounds__(1024) void k_scene_prep_one(JobBufs b) {
-    __shared__ uint32_t l1[16], l2[16];
-    const bool bad = b.cnt->overflow != 0;  // from the earlier kernels
-    const uint32_t total = scan_one<uint32_t>(b.nsub, scan_len(b.tri_cap, &b.head->ntri), b.suboff,
-                                              &b.cnt->nprims_raw, l1);
-    __syncthreads();
-    const uint2 cm = scene_prep(b, total, l1, l2);
-    // the prim slots and the coarse matrix fit (the overflow bits scene_prep sets)
-    const bool fits = (uint64_t)cm.x * CHUNK <= b.prim_cap && cm.y <= b.mat_cap;
-    __syncthreads();
-    if (!bad && fits) pchunk_map(b, cm.x);
+    constexpr uint32_t PER = 4;  // chunks per thread and pass
+    const uint32_t nc = min(b.head->ntri / TRI_ALIGN, b.tchunk_cap);
+    const uint4* prims = reinterpret_cast<const uint4*>(b.wave_prims);  // a chunk's four waves
+    uint32_t total = 0;
+    uint4 w[PER];  // each pass's counts are asked for one pass ahead
+    auto fetch = [&](uint32_t c0) {
+        for (uint32_t i = 0; i < PER; ++i) w[i] = c0 + i < nc ? prims[c0 + i] : make_uint4(0u, 0u, 0u, 0u);
+    };
+    uint32_t c0 = threadIdx.x * PER;
+    fetch(c0);
+    for (uint32_t base = 0; base < nc; base += 1024u * PER, c0 += 1024u * PER) {
+        uint32_t v[PER], s = 0;
+        for (uint32_t i = 0; i < PER; ++i) {
+            v[i] = w[i].x + w[i].y + w[i].z + w[i].w;
+            s += v[i];
+        }
+        fetch(c0 + 1024u * PER);
+        uint32_t tot;
+        uint32_t ex = total + block_exclusive_scan<uint32_t>(s, l1, &tot);
+        for (uint32_t i = 0; i < PER; ++i) {
+            if (c0 + i < nc) b.chunk_off[c0 + i] = ex;
+            ex += v[i];
+        }
+        total += tot;
+    }
+    if (threadIdx.x == 0) b.cnt->nprims_raw = total;
+    __syncthreads();  // orders the offsets before their use
+    scene_prep(b, total, l1, l2);
 }
 
 // ---------------------------------------------------------------------------
-// k_setup: one thread per input triangle; writes its rasterizer triangles
-// at the scene's prim slots in fan order.
+// k_setup: one thread per rasterizer triangle of a 256-triangle chunk; written
+// at the scene's prim slots in (triangle, fan) order.
 // mod.rs:284-313 (divide), mod.rs:315-345 (viewport), mod.rs:187-222 (edge
 // setup), bounding_box.rs:13-42 + mod.rs:347-361 (clamped pixel bbox).
 // Besides the reference's values each prim carries derived, exactly
@@ -885,23 +874,23 @@ constexpr uint32_t SETUP_STAGE = 336;
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_setup(
     JobBufs b, const DrawDev* __restrict__ draws, const SceneCfg* __restrict__ scenes,
     const SceneRun* __restrict__ runs, const uint32_t* __restrict__ tchunk_draw,
-    const uint32_t* __restrict__ suboff, const uint32_t* __restrict__ nsub, const uint32_t* __restrict__ cls,
+    const uint32_t* __restrict__ chunk_off, const uint32_t* __restrict__ nsub, const uint32_t* __restrict__ cls,
     const float* __restrict__ clip_out) {
     __shared__ PrimGeom stage[SETUP_STAGE];
     __shared__ uint32_t poff[256], pcls[256];  // per triangle of the chunk: first prim (chunk-relative), class
+    __shared__ uint32_t wtot[4];               // per wave of the chunk: its prims
     if (uniform(b.cnt->overflow) != 0) return;
     const uint32_t NT = b.head->ntri;
     const uint32_t prim_cap = b.prim_cap;
     // the chunk table words of the workgroup's next chunk are loaded one
-    // chunk ahead (NT is a multiple of 256, so t0 + 255 is in range)
-    uint32_t n_d = 0, n_s0 = 0, n_end = 0, n_sub = 0, n_cls = 0;
+    // chunk ahead (NT is a multiple of 256)
+    uint32_t n_d = 0, n_s0 = 0, n_sub = 0, n_cls = 0;
     auto fetch = [&](uint32_t c) {
         if (c * 256u < NT) {
             const uint32_t c0 = c * 256u;
             n_d = tchunk_draw[c];
-            n_s0 = suboff[c0];
-            n_end = suboff[c0 + 255u] + nsub[c0 + 255u];
-            n_sub = suboff[c0 + threadIdx.x];
+            n_s0 = chunk_off[c];
+            n_sub = nsub[c0 + threadIdx.x];
             n_cls = cls[c0 + threadIdx.x];
         }
     };
@@ -909,7 +898,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     for (uint32_t blk = blockIdx.x; blk * 256u < NT; blk += gridDim.x) {
         const uint32_t t0 = blk * 256u;
         const uint32_t t = t0 + threadIdx.x;
-        const uint32_t d = uniform(n_d), s0 = uniform(n_s0), s_end = uniform(n_end), my_sub = n_sub, my_cls = n_cls;
+        const uint32_t d = uniform(n_d), s0 = uniform(n_s0), my_cls = n_cls;
+        const uint32_t my_prims = my_cls < 2u ? my_cls : min(n_sub, MAXV - 2u);
         fetch(blk + gridDim.x);
         const DrawDev& dd = draws[d];
         const uint32_t scene = dd.scene;
@@ -921,11 +911,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         const bool proofs = b.exact_paths == 0;
         // the chunk's prim range (its 256 triangles belong to draw d: draws are 256-aligned)
         const uint32_t blk_first = uniform(run.prim_base + (s0 - run.prim_off));
-        const uint32_t nblk = s_end - s0;
+        // each triangle's first prim: prefix sum of the counts (below 16: four
+        // bit planes) over the wave, then over the waves
+        uint32_t pre = 0, mine = 0;
+        for (uint32_t bit = 0; bit < 4; ++bit) {
+            const uint64_t m = ballot((my_prims >> bit) & 1u);
+            pre += mbcnt(m) << bit;
+            mine += (uint32_t)__popcll(m) << bit;
+        }
+        const uint32_t wave = threadIdx.x >> 6;
+        if (lane_id() == 0) wtot[wave] = mine;
+        pcls[threadIdx.x] = (t - dd.tri_base < dd.ntri) ? my_cls : 0u;
+        __syncthreads();
+        const uint32_t t1 = wtot[0], t2 = t1 + wtot[1], t3 = t2 + wtot[2];
+        const uint32_t nblk = uniform(t3 + wtot[3]);
+        poff[threadIdx.x] = pre + (wave == 0 ? 0u : wave == 1 ? t1 : wave == 2 ? t2 : t3);
         const uint32_t blk_end = blk_first + nblk;
         const bool staged = nblk <= SETUP_STAGE && blk_end <= prim_cap;
-        poff[threadIdx.x] = my_sub - s0;
-        pcls[threadIdx.x] = (t - dd.tri_base < dd.ntri) ? my_cls : 0u;
+        // the scene of each binning chunk that starts among these prims
+        const uint32_t bc = (blk_first + CHUNK - 1u) / CHUNK + threadIdx.x;
+        if (bc * CHUNK < blk_end && bc < b.pchunk_cap) b.pchunk_scene[bc] = scene;
         __syncthreads();
         // one thread per prim of the chunk: an input triangle (class 1) or one
         // fan triangle of a clipped polygon (class 2 + slot), so clipped
@@ -2753,14 +2758,8 @@ void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_s
     k_job_init<<<at_least1(g.init), 256, 0, s>>>(b);
     k_classify<<<at_least1(std::min<uint32_t>(g.tris, 2048u)), 256, 0, s>>>(b, b.tchunk_draw, b.draws);
     k_clip<<<at_least1((g.clip + CLIP_GROUPS - 1) / CLIP_GROUPS), 64, 0, s>>>(b);
-    if (b.tri_cap <= SCAN_ONE_MAX) {
-        k_scene_prep_one<<<1, 1024, 0, s>>>(b);
-    } else {
-        launch_scan<uint32_t>(s, b.nsub, b.suboff, b.tri_cap, &b.head->ntri, b.parts, &b.cnt->nprims_raw);
-        k_scene_prep<<<1, 1024, 0, s>>>(b);
-        k_pchunk_map<<<at_least1(std::min<uint32_t>(g.bins / 256 + 1, 1024u)), 256, 0, s>>>(b);
-    }
-    k_setup<<<at_least1(g.tris), 256, 0, s>>>(b, b.draws, b.scenes, b.runs, b.tchunk_draw, b.suboff, b.nsub, b.cls,
+    k_scene_prep<<<1, 1024, 0, s>>>(b);
+    k_setup<<<at_least1(g.tris), 256, 0, s>>>(b, b.draws, b.scenes, b.runs, b.tchunk_draw, b.chunk_off, b.nsub, b.cls,
                                               b.clip_out);
     if (ev_bin) (void)hipEventRecord(ev_bin, s);
     k_bin<false><<<at_least1(g.bins), 256, 0, s>>>(b, b.pchunk_scene, b.scenes, b.runs, b.pbin, b.bin_offsets);
