@@ -207,9 +207,11 @@ int rz_batch_scene_flags(const rz_ctx *ctx, uint32_t scene, uint32_t *flags);
 /* Batch tuning: bin_target = most coarse bins per scene when choosing the
  * bin side automatically (1..256); raster_per_cu = persistent raster
  * workgroups per CU (0: one single-wave workgroup per 8x8 quadrant);
- * use_graph = replay the captured HIP graph (1) or launch the kernels
- * directly (0), for batches and for frames of at most 65536 triangles
- * (while profiling is on, frames launch directly). Between jobs. */
+ * use_graph = replay a captured HIP graph where that is the faster (1:
+ * batches with a scene of more than 16384 triangles or of great extent, and
+ * frames of at most 65536 triangles that are read back to the host; while
+ * profiling is on, frames launch directly) or always launch the kernels
+ * directly (0). Between jobs. */
 int rz_batch_tuning(rz_ctx *ctx, uint32_t bin_target, uint32_t raster_per_cu, int use_graph);
 /* The current tuning: [bin_target, raster_per_cu, use_graph]. */
 int rz_batch_get_tuning(const rz_ctx *ctx, uint32_t out[3]);

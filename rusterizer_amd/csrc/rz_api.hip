@@ -114,9 +114,20 @@ struct JobPlan {
     uint32_t ntri = 0, ntiles = 0, nbins = 0;
     uint32_t max_nb = 1, max_T = 1;
     uint64_t tris = 0;  // input triangles
+    bool direct = false;   // binned by k_tile_bin
+    uint32_t nftiles = 0;  // 32x32 tiles
 };
 
 enum class JobKind { None, Frame, Batch };
+
+// a captured launch sequence and what it was captured for
+struct JobGraph {
+    hipGraphExec_t exec = nullptr;
+    uint64_t gen = ~0ull;
+    uint32_t dcap = 0, scap = 0, raster = 0, tiles = 0;
+    bool stats = false;
+    int svc = -1;  // the raster service entry it posts to
+};
 
 }  // namespace
 
@@ -180,12 +191,10 @@ struct rz_ctx {
     DBuf<float> msaa_depth;
     uint64_t gen = 0;  // bumped whenever a buffer moves (invalidates the graph)
 
-    // graph of the batch launch sequence
-    hipGraphExec_t graph = nullptr;
-    uint64_t graph_gen = ~0ull;
-    uint32_t graph_dcap = 0, graph_scap = 0, graph_raster = 0, graph_tiles = 0;
-    uint32_t tiles_cap = 0;  // raster grid of the graph: most tiles of any job so far
-    bool graph_stats = false;
+    // graphs of the launch sequence: with coarse and fine binning, and with
+    // k_tile_bin (a context that serves jobs of both kinds keeps both)
+    JobGraph graphs[2];
+    uint32_t tiles_cap = 0;  // raster grid of the graphs: most tiles of any job so far
 
     hipEvent_t done = nullptr;
     uint32_t replays = 0, ovf_seen = 0;
@@ -193,7 +202,6 @@ struct rz_ctx {
 
     // raster service (rz_service_attach): this context's entry, or -1
     int svc_entry = -1;
-    int graph_svc = -1;    // the entry the captured graph posts to
     bool job_svc = false;  // the job in flight was posted to the service
     uint32_t job_gen = 0;  // its number
 
@@ -283,6 +291,28 @@ void scene_bins(uint32_t W, uint32_t H, uint32_t req_cb, uint32_t target, uint32
     }
 }
 
+// Whether a job is binned by k_tile_bin: no scene beyond its bit masks, and
+// tiles times triangles (each tile costs as much as 1024 more) so few that
+// looking at every prim from every tile takes less than the two-level binning's
+// launches. Both, in us a frame (work in millions): 1280x720, 4,000 triangles
+// (4.6) 93 direct, 117 two-level; 16,000 (15.7) 120, 137; 1920x1080, 4,000
+// (10.2) 119, 129; 16,000 (34.7) 157, 158; 3840x2160, 300 (10.8) 121, 146; 1,500
+// (20.6) 184, 171; 32 scenes of 256-512 px (19) 283, 275.
+constexpr uint64_t DIRECT_WORK = 16ull << 20;
+constexpr uint64_t DIRECT_TILE = 1024;
+
+struct DirectRule {
+    uint64_t work = 0, ftiles = 0;
+    bool fits = true;
+    void scene(uint32_t W, uint32_t H, uint64_t tris) {
+        const uint64_t ft = (uint64_t)((W + 31) / 32) * ((H + 31) / 32);
+        ftiles += ft;
+        work += ft * (tris + DIRECT_TILE);
+        fits = fits && tris <= DIRECT_TRIS;
+    }
+    bool direct() const { return fits && work <= DIRECT_WORK && ftiles <= 0xFFFF0000ull; }
+};
+
 uint32_t clamp_u32(uint64_t v) { return v > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)v; }
 
 // table block layout at capacities (dcap draws, scap scenes)
@@ -340,6 +370,7 @@ int build_job(rz_ctx* c, JobPlan& pl) {
     uint32_t d = 0;
     std::vector<double>& dens = c->scene_density;  // input triangles per pixel, for the raster order
     dens.assign(ns, 0.0);
+    DirectRule rule;
     for (uint32_t s = 0; s < ns; ++s) {
         const PendingScene& ps = c->scenes[s];
         SceneCfg& g = sc[s];
@@ -388,6 +419,8 @@ int build_job(rz_ctx* c, JobPlan& pl) {
         }
         g.tri_end = (uint32_t)tri;
         g.draw = d - first_draw == 1 ? first_draw : MANY_DRAWS;
+        g.ftile_base = (uint32_t)rule.ftiles;
+        rule.scene(ps.W, ps.H, (uint64_t)dens[s]);
         tiles += (uint64_t)((ps.W + 15) / 16) * ((ps.H + 15) / 16);
         bins += (uint64_t)g.nbx * g.nby;
         pl.max_nb = std::max(pl.max_nb, g.nbx * g.nby);
@@ -397,6 +430,10 @@ int build_job(rz_ctx* c, JobPlan& pl) {
     if (tiles > 0xFFFF0000ull || bins > 0xFFFF0000ull) return fail(c, RZ_ERR_LIMIT, "job too large");
     // raster order: the scenes' tile ranges densest first (ties in scene
     // order), so that the longest tiles do not trail at the end of the launch
+    pl.direct = rule.direct();
+    pl.nftiles = clamp_u32(rule.ftiles);
+    if (pl.direct)  // the lists are of 32x32 tiles, whatever side was asked for
+        for (uint32_t s = 0; s < ns; ++s) sc[s].fts = 5;
     std::vector<uint32_t>& order = c->scene_order;
     order.resize(ns);
     for (uint32_t s = 0; s < ns; ++s) {
@@ -418,6 +455,7 @@ int build_job(rz_ctx* c, JobPlan& pl) {
     head->ntri = pl.ntri;
     head->ntiles = pl.ntiles;
     head->nbins = pl.nbins;
+    head->nftiles = pl.nftiles;
     return RZ_OK;
 }
 
@@ -475,21 +513,22 @@ int size_buffers(rz_ctx* c, const JobPlan& pl, const Needs& n_in, G& g) {
     g(c->uvat, geom * UV_STRIDE);
     g(c->pbin, geom);
     g(c->tchunk_draw, cls / TRI_ALIGN + 1);
-    g(c->pchunk_scene, geom / CHUNK + 1);
+    g(c->tile_rec, 4 * std::max<uint64_t>(pl.ntiles, 1));
+    g(c->flist, n.fine);
     if (c->raster_stats) g(c->rstat_parts, 5ull * (4ull * pl.ntiles + 512 + 32ull * (uint32_t)c->n_cu));
     const size_t clip = g(c->clip_tri, n.clip);
     g(c->clip_draw, clip);
     g(c->clip_out, clip * MAXV * 10);
+    if (pl.direct) return g.rc;  // k_tile_bin needs none of the two-level binning's buffers
+    g(c->pchunk_scene, geom / CHUNK + 1);
     const size_t list = g(c->list, n.pairs);
     // coarse matrix: sum over scenes of bins * chunks <= max_nb * (slots / CHUNK)
     const uint64_t mat = std::max<uint64_t>(n.mat, (uint64_t)pl.max_nb * (geom / CHUNK + 1));
     const size_t mat_cap = g(c->bin_counts, mat);
     g(c->bin_offsets, mat_cap);
     const size_t bins = g(c->bin_rng, std::max<uint64_t>(pl.nbins, 1));
-    g(c->tile_rec, 4 * std::max<uint64_t>(pl.ntiles, 1));
     g(c->fpack, bins);
     g(c->fpre, bins);
-    g(c->flist, n.fine);
     // fine-binning chunks: sum over bins of ceil(len / CHUNK) <= entries / CHUNK + bins
     g(c->fchunk_rec, list / CHUNK + bins + 1);
     // fine matrix: sum over bins of T * ceil(len / CHUNK) <= max_T * (entries / CHUNK + bins)
@@ -510,12 +549,15 @@ int ensure_buffers(rz_ctx* c, const JobPlan& pl, const Needs& n_in) {
 
 // Sizes of a job (no tables written): draw(i) gives the triangle count of
 // draw i, scene(i, W, H) the size of scene i.
-template <class DrawTris, class SceneSize>
-void plan_sizes(const rz_ctx* c, bool frame, uint32_t nd, uint32_t ns, DrawTris draw, SceneSize scene, JobPlan& pl) {
+// (scene_tris: the triangles of scene i's draws)
+template <class DrawTris, class SceneSize, class SceneTris>
+void plan_sizes(const rz_ctx* c, bool frame, uint32_t nd, uint32_t ns, DrawTris draw, SceneSize scene,
+                SceneTris scene_tris, JobPlan& pl) {
     pl = JobPlan{};
     pl.ndraws = nd;
     pl.nscenes = ns;
     uint64_t tri = 0, tiles = 0, bins = 0;
+    DirectRule rule;
     for (uint32_t i = 0; i < nd; ++i) {
         const uint32_t n = draw(i);
         tri += ((uint64_t)n + TRI_ALIGN - 1) / TRI_ALIGN * TRI_ALIGN;
@@ -533,7 +575,10 @@ void plan_sizes(const rz_ctx* c, bool frame, uint32_t nd, uint32_t ns, DrawTris 
         bins += nb;
         pl.max_nb = std::max(pl.max_nb, nb);
         pl.max_T = std::max(pl.max_T, (cb >> fts) * (cb >> fts));
+        rule.scene(W, H, scene_tris(i));
     }
+    pl.direct = rule.direct();
+    pl.nftiles = clamp_u32(rule.ftiles);
     pl.ntri = clamp_u32(tri);
     pl.ntiles = clamp_u32(tiles);
     pl.nbins = clamp_u32(bins);
@@ -541,6 +586,9 @@ void plan_sizes(const rz_ctx* c, bool frame, uint32_t nd, uint32_t ns, DrawTris 
 
 // The plan of the recorded scenes and draws.
 void plan_job(const rz_ctx* c, JobPlan& pl) {
+    std::vector<uint64_t> tris(c->scenes.size(), 0);
+    for (const PendingDraw& d : c->draws)
+        if (d.scene < tris.size()) tris[d.scene] += d.mesh->ntri;
     plan_sizes(
         c, c->recording == JobKind::Frame, (uint32_t)c->draws.size(), (uint32_t)c->scenes.size(),
         [&](uint32_t i) { return c->draws[i].mesh->ntri; },
@@ -548,7 +596,7 @@ void plan_job(const rz_ctx* c, JobPlan& pl) {
             W = c->scenes[i].W;
             H = c->scenes[i].H;
         },
-        pl);
+        [&](uint32_t i) { return tris[i]; }, pl);
 }
 
 template <class T>
@@ -622,7 +670,7 @@ JobBufs job_bufs(const rz_ctx* c) {
     b.clip_cap = clamp_u32(c->clip_tri.cap);
     b.prim_cap = clamp_u32(c->geom.cap);
     b.pair_cap = clamp_u32(c->list.cap);
-    b.mat_cap = clamp_u32(c->bin_counts.cap);
+    b.mat_cap = c->plan.direct ? ~0u : clamp_u32(c->bin_counts.cap);  // k_tile_bin has no count matrices
     b.fine_cap = clamp_u32(c->flist.cap);
     b.fmat_cap = clamp_u32(c->fine_counts.cap);
     b.bins_cap = clamp_u32(c->bin_rng.cap);
@@ -633,6 +681,7 @@ JobBufs job_bufs(const rz_ctx* c) {
     b.rstat_cap = clamp_u32(c->rstat_parts.cap / 5);
     b.clip_wide = c->clip_wide ? 1u : 0u;
     b.exact_paths = c->exact_paths ? 1u : 0u;
+    b.direct = c->plan.direct ? 1u : 0u;
     return b;
 }
 
@@ -737,6 +786,8 @@ JobGrid job_grid(const rz_ctx* c, const JobPlan& pl, bool for_graph) {
     g.fine = (uint32_t)std::min<uint64_t>(fch, 8192);
     g.raster = c->raster_per_cu ? c->raster_per_cu * (uint32_t)c->n_cu : 0;
     g.ntiles = for_graph ? std::max(c->tiles_cap, pl.ntiles) : pl.ntiles;
+    // (a graph's: 32x32 tiles are at least a quarter of the 16x16 ones)
+    if (pl.direct) g.direct = std::max(1u, std::min<uint32_t>(for_graph ? (g.ntiles + 2) / 3 : pl.nftiles, 8192));
     return g;
 }
 
@@ -768,13 +819,13 @@ int enqueue_graph(rz_ctx* c, const JobPlan& pl) {
     const int svc = c->job_svc ? c->svc_entry : -1;
     if (pl.ntiles > c->tiles_cap) c->tiles_cap = std::max<uint32_t>(pl.ntiles, c->tiles_cap + c->tiles_cap / 4);
     const JobGrid g = job_grid(c, pl, true);
-    if (!c->graph || c->graph_gen != c->gen || c->graph_dcap != c->dcap || c->graph_scap != c->scap ||
-        c->graph_raster != g.raster || c->graph_tiles != g.ntiles || c->graph_stats != c->raster_stats ||
-        c->graph_svc != svc) {
-        if (c->graph) {
+    JobGraph& jg = c->graphs[pl.direct ? 1 : 0];
+    if (!jg.exec || jg.gen != c->gen || jg.dcap != c->dcap || jg.scap != c->scap || jg.raster != g.raster ||
+        jg.tiles != g.ntiles || jg.stats != c->raster_stats || jg.svc != svc) {
+        if (jg.exec) {
             HIP_TRY(c, hipStreamSynchronize(s));
-            (void)hipGraphExecDestroy(c->graph);
-            c->graph = nullptr;
+            (void)hipGraphExecDestroy(jg.exec);
+            jg.exec = nullptr;
         }
         hipGraph_t graph = nullptr;
         HIP_TRY(c, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -788,22 +839,22 @@ int enqueue_graph(rz_ctx* c, const JobPlan& pl) {
             if (graph) (void)hipGraphDestroy(graph);
             return fail(c, RZ_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e != hipSuccess ? e : e2));
         }
-        e = hipGraphInstantiate(&c->graph, graph, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(&jg.exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (e != hipSuccess) {
-            c->graph = nullptr;
+            jg.exec = nullptr;
             return fail(c, RZ_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
         }
-        c->graph_gen = c->gen;
-        c->graph_dcap = c->dcap;
-        c->graph_scap = c->scap;
-        c->graph_raster = g.raster;
-        c->graph_tiles = g.ntiles;
-        c->graph_stats = c->raster_stats;
-        c->graph_svc = svc;
+        jg.gen = c->gen;
+        jg.dcap = c->dcap;
+        jg.scap = c->scap;
+        jg.raster = g.raster;
+        jg.tiles = g.ntiles;
+        jg.stats = c->raster_stats;
+        jg.svc = svc;
     }
     if (c->prof) HIP_TRY(c, hipEventRecord(c->ev[0], s));
-    HIP_TRY(c, hipGraphLaunch(c->graph, s));
+    HIP_TRY(c, hipGraphLaunch(jg.exec, s));
     if (c->prof) HIP_TRY(c, hipEventRecord(c->ev[3], s));
     HIP_TRY(c, hipEventRecord(c->done, s));
     c->job_graph = true;
@@ -895,22 +946,26 @@ int complete_job(rz_ctx* c) {
     return 1;
 }
 
-// graph: replay the captured graph for jobs of at most graph_max_tris input
-// triangles, launch directly otherwise
-int start_job(rz_ctx* c, bool graph, uint64_t graph_max_tris = ~0ull) {
+// graph(plan): whether to replay the captured graph or to launch directly
+template <class Graph>
+int start_job(rz_ctx* c, Graph graph) {
     int rc = build_job(c, c->plan);
     if (rc) return rc;
     c->replays = 0;
     c->ovf_seen = 0;
     c->in_flight = true;
-    return enqueue(c, graph && c->plan.tris <= graph_max_tris);
+    return enqueue(c, c->use_graph && graph(c->plan));
 }
 
-// Frames of at most this many input triangles replay the captured graph: one
-// submission instead of a launch per kernel, for frames whose time is the
-// host's launches (a 12-triangle cube frame: mean 0.115 -> 0.103 ms, p99
-// 0.19 -> 0.11 ms). Larger frames launch directly: the graph's grids, sized
-// to the buffer capacities, made a 1M-triangle frame about 1% slower.
+// Frames that are read back to the host and have at most this many input
+// triangles replay the captured graph: the launches that follow a copy to
+// pageable memory cost the host more (cube at 800x600 read back: graph 0.194,
+// direct 0.211 ms). Frames left on the device launch directly, their grids
+// exact and their seven kernels cheaper to launch than the graph (3,001
+// triangles at 641x479: direct 0.077, graph 0.085 ms; 60,000 at 1279x719: 0.174
+// against 0.182 ms), and so do batches binned by k_tile_bin (one scene of 15,000
+// triangles 0.099 against 0.108 ms; 300 thumbnails 0.330 against 0.346 ms).
+// Other batches replay the graph.
 constexpr uint64_t FRAME_GRAPH_TRIS = 65536;
 
 int wait_job(rz_ctx* c) {
@@ -945,9 +1000,9 @@ int frame_impl(rz_ctx* c, uint32_t* host_out, uint32_t* dev_out, uint32_t* host_
     c->scenes.clear();
     c->scenes.push_back(PendingScene{c->W, c->H, c->clear_depth, target, want_msaa ? c->msaa_color.p : nullptr,
                                      want_msaa ? c->msaa_depth.p : nullptr});
-    // small frames replay the captured graph; direct launches while
-    // profiling, whose stage events sit between the kernels
-    rc = start_job(c, c->use_graph && !c->prof, FRAME_GRAPH_TRIS);
+    // direct launches while profiling, whose stage events sit between the kernels
+    const bool read_back = host_out || host_color4 || host_depth4;
+    rc = start_job(c, [&](const JobPlan& pl) { return read_back && !c->prof && pl.tris <= FRAME_GRAPH_TRIS; });
     if (!rc) rc = wait_job(c);
     release_job(c);
     c->clear_depth = c->next_clear_depth;
@@ -1406,7 +1461,8 @@ int rz_destroy(rz_ctx* c) {
     if (c->svc_entry >= 0) c->pool->svc.used &= ~(1u << c->svc_entry);
     for (PendingDraw& d : c->draws) d.mesh->pending--;
     c->draws.clear();
-    if (c->graph) (void)hipGraphExecDestroy(c->graph);
+    for (JobGraph& jg : c->graphs)
+        if (jg.exec) (void)hipGraphExecDestroy(jg.exec);
     release(c->cls);
     release(c->nsub);
     release(c->wave_prims);
@@ -1623,10 +1679,11 @@ int rz_trim(rz_ctx* c) {
     if (c->recording != JobKind::None || c->in_flight || !c->draws.empty())
         return fail(c, RZ_ERR_STATE, "not between jobs");
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (c->graph) {
-        (void)hipGraphExecDestroy(c->graph);
-        c->graph = nullptr;
-    }
+    for (JobGraph& jg : c->graphs)
+        if (jg.exec) {
+            (void)hipGraphExecDestroy(jg.exec);
+            jg.exec = nullptr;
+        }
     release(c->cls);
     release(c->nsub);
     release(c->wave_prims);
@@ -1674,7 +1731,7 @@ int rz_batch_need(const rz_ctx* c, const rz_batch_item* items, uint32_t n, uint6
             W = items[i].width;
             H = items[i].height;
         },
-        pl);
+        [&](uint32_t i) { return (uint64_t)items[i].mesh->ntri; }, pl);
     *bytes = n ? job_bytes_after(c, pl) : ctx_bytes(c);
     return RZ_OK;
 }
@@ -1807,7 +1864,7 @@ int rz_batch_submit(rz_ctx* c) {
     // group draws by scene, keeping each scene's submission order
     std::stable_sort(c->draws.begin(), c->draws.end(),
                      [](const PendingDraw& a, const PendingDraw& b) { return a.scene < b.scene; });
-    int rc = start_job(c, c->use_graph);
+    int rc = start_job(c, [](const JobPlan& pl) { return !pl.direct; });
     if (rc) {
         release_job(c);
         return rc;

@@ -25,6 +25,11 @@ constexpr uint32_t MAX_BINS = 256;    // coarse bins per scene (one binning thre
 constexpr uint32_t TRI_ALIGN = 256;   // draws start at multiples of this in the triangle index space
 constexpr uint32_t ATTR_STRIDE = 12;  // floats of colour attributes per prim (3 x RGBA)
 constexpr uint32_t UV_STRIDE = 6;     // floats of texture coordinates per prim (3 x uv)
+// Jobs whose scenes have at most DIRECT_TRIS input triangles each can be binned
+// by k_tile_bin, which keeps a bit per prim of a scene in LDS (a clipped
+// triangle gives at most MAXV - 2 prims)
+constexpr uint32_t DIRECT_TRIS = 16384;
+constexpr uint32_t DIRECT_WORDS = DIRECT_TRIS / 64 * (MAXV - 2);
 constexpr int SCAN_ITEMS = 8;
 constexpr uint32_t SCAN_TILE = 256 * SCAN_ITEMS;
 constexpr uint32_t NO_TILE = 0xFFFFFFFFu;
@@ -69,7 +74,8 @@ struct JobHead {
     uint32_t ntiles;  // 16x16 raster tiles of all scenes
     uint32_t nbins;   // coarse bins of all scenes
     uint32_t svc_gen;  // raster service: number of this job in its context (low 16 bits are posted)
-    uint32_t pad[2];
+    uint32_t nftiles;  // 32x32 tiles of all scenes
+    uint32_t pad;
 };
 
 // Per-draw state on the device (mesh streams, fragment shader, MVP).
@@ -105,7 +111,7 @@ struct SceneCfg {
     uint32_t* msaa_color;     // optional W*H*4 pre-resolve colours
     float* msaa_depth;        // optional W*H*4 pre-resolve depths
     uint32_t draw;            // the scene's only draw, or MANY_DRAWS
-    uint32_t pad2;
+    uint32_t ftile_base;      // first global 32x32 tile of the scene (jobs binned by k_tile_bin)
 };
 static_assert(sizeof(SceneCfg) == 80, "SceneCfg layout");
 
@@ -155,7 +161,8 @@ struct JobBufs {
     // geometry
     uint32_t* cls;
     uint32_t* nsub;       // rasterizer triangles of each clipped triangle
-    uint32_t* wave_prims; // rasterizer triangles of each 64 triangles
+    uint32_t* wave_prims; // rasterizer triangles of each 64 triangles; with direct, k_setup leaves its
+                          // waves' coarse entries here
     uint32_t* chunk_off;  // per TRI_ALIGN-triangle chunk: the rasterizer triangles of all earlier ones
     uint32_t* clip_tri;   // clipped triangle of each clip slot
     uint32_t* clip_draw;  // its draw
@@ -188,6 +195,7 @@ struct JobBufs {
     uint32_t tile_cap;  // raster tiles tile_rec holds (4 records each)
     uint32_t tchunk_cap, pchunk_cap, rstat_cap;  // rstat_cap in workgroups
     uint32_t clip_wide;    // clip every polygon with a full wave
+    uint32_t direct;       // binned by k_tile_bin
     uint32_t exact_paths;  // setup proves nothing: every prim takes the raster's exact paths
     uint32_t* svc_flags;   // raster service: pinned host array of the scenes' final flags
     // the job tables as the host wrote them (pinned host memory, or the
@@ -219,6 +227,7 @@ struct JobGrid {
     uint32_t fine;       // k_fine_bin blocks
     uint32_t raster;     // persistent raster workgroups; 0 = one one-wave workgroup per quadrant
     uint32_t ntiles;     // tiles the one-per-tile raster grid must cover (>= the job's)
+    uint32_t direct;     // k_tile_bin blocks; 0 = coarse and fine binning
 };
 
 // A block of words passed to a kernel by value (kernel arguments hold up to

@@ -12,6 +12,7 @@
 //   -> k_fine_prep -> scan64 -> k_fine_bin<count> -> scan
 //   -> k_fine_bin<scatter>                      (8, 16 or 32 px fine tiles)
 //   -> k_tile_prep -> k_raster_q (coverage, depth, shading, resolve)
+// (small jobs: k_tile_bin in place of both binning levels and k_tile_prep)
 // Rasterizer triangles ("prims") are stored per scene in submission order
 // (draw, input triangle, clip-fan index), so every later stage keeps the
 // reference's order per pixel without sorting. Each scene's prims start at a
@@ -791,7 +792,15 @@ __device__ __forceinline__ bool finite_bary(const PrimGeom& o) {
     return ok;
 }
 
-__device__ __forceinline__ void setup_prim(const ClipV* tv, uint32_t W, uint32_t H, uint32_t draw, uint32_t fs,
+// coarse bins along one axis that the bbox side lo | hi << 16 covers (see k_setup)
+__device__ __forceinline__ uint32_t bins_covered(uint32_t side, uint32_t per_bin) {
+    const uint32_t lo = side & 0xFFFFu, hi = side >> 16;
+    if (lo >= hi) return 0u;
+    return ((((hi - 1u) >> 4) * per_bin) >> 16) - (((lo >> 4) * per_bin) >> 16) + 1u;
+}
+
+// (returns the prim's pixel bbox)
+__device__ __forceinline__ uint2 setup_prim(const ClipV* tv, uint32_t W, uint32_t H, uint32_t draw, uint32_t fs,
                                            bool tex_idx32, bool proofs, PrimGeom* g, float* __restrict__ attr,
                                            float* __restrict__ uvat, uint4* __restrict__ pbin) {
     const float zmin = 0.0f, zmax = 1.0f;
@@ -860,6 +869,7 @@ __device__ __forceinline__ void setup_prim(const ClipV* tv, uint32_t W, uint32_t
         a2[1] = make_float2(tv[1].a[4], tv[1].a[5]);
         a2[2] = make_float2(tv[2].a[4], tv[2].a[5]);
     }
+    return make_uint2(x0 | (x1 << 16), y0 | (y1 << 16));
 }
 
 // The prims of a workgroup's 256 triangles are one contiguous range; when it
@@ -932,6 +942,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         const uint32_t bc = (blk_first + CHUNK - 1u) / CHUNK + threadIdx.x;
         if (bc * CHUNK < blk_end && bc < b.pchunk_cap) b.pchunk_scene[bc] = scene;
         __syncthreads();
+        // with direct binning: the coarse bins the thread's prims cover (x / cb
+        // = (x / 16) * (65536 / (cb / 16) + 1) >> 16 for x below 2^14)
+        const uint32_t per_bin = b.direct ? 65536u / (sc.cb >> 4) + 1u : 0u;
+        uint32_t pairs = 0;
         // one thread per prim of the chunk: an input triangle (class 1) or one
         // fan triangle of a clipped polygon (class 2 + slot), so clipped
         // triangles' fans spread over the workgroup
@@ -963,11 +977,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                     for (int i = 0; i < 6; ++i) tv[q].a[i] = pv[4 + i];
                 }
             }
-            if (prim < prim_cap)
-                setup_prim(tv, W, H, d, fs, tex_idx32, proofs, staged ? stage + pp : b.geom + prim,
-                           b.attrs + (size_t)prim * ATTR_STRIDE, b.uvat + (size_t)prim * UV_STRIDE, b.pbin + prim);
-            else
+            if (prim < prim_cap) {
+                const uint2 bb = setup_prim(tv, W, H, d, fs, tex_idx32, proofs, staged ? stage + pp : b.geom + prim,
+                                            b.attrs + (size_t)prim * ATTR_STRIDE, b.uvat + (size_t)prim * UV_STRIDE,
+                                            b.pbin + prim);
+                if (per_bin != 0) pairs += bins_covered(bb.x, per_bin) * bins_covered(bb.y, per_bin);
+            } else {
                 ovf = true;
+            }
+        }
+        if (per_bin != 0) {
+            for (int o = 32; o >= 1; o >>= 1) pairs += (uint32_t)__shfl_xor((int)pairs, o);
+            if (lane_id() == 0) b.wave_prims[blk * 4u + wave] = pairs;
         }
         __syncthreads();
         if (staged) {
@@ -1382,6 +1403,110 @@ __global__ __launch_bounds__(256) void k_tile_prep(JobBufs b) {
         const uint32_t lbeg = min(s_idx < fmat_len ? b.fine_off[s_idx] : ftot, lend);
         const uint32_t slot = sc.raster_base + blocked_rank(tx, ty, ntx, nty);
         if (slot < b.tile_cap) b.tile_rec[4u * slot + q] = make_uint4(s, lbeg, lend, px | py << 16);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// k_tile_bin: binning of jobs with few prims per scene, in one launch instead of
+// the eight of the two-level binning. A workgroup takes a 32x32 tile and looks
+// at every prim of the tile's scene, a bit each in LDS; the set bits, in prim
+// order, are the tile's list, whose place it reserves with one atomic. The work
+// grows as tiles times prims, all of it 16-byte reads that stay in L2, where the
+// eight launches take about 35 us however small the job; the host's rule
+// (direct_binning) draws the line. Tile records are written here too.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t find_scene_ftile(const SceneCfg* __restrict__ sc, uint32_t ns, uint32_t t) {
+    uint32_t lo = 0, hi = ns;
+    while (hi - lo > 1) {
+        uint32_t mid = (lo + hi) >> 1;
+        if (sc[mid].ftile_base <= t) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __restrict__ pbin,
+                                                  const SceneCfg* __restrict__ scenes,
+                                                  const SceneRun* __restrict__ runs) {
+    constexpr uint32_t ROUND = 2048;  // entries written per round
+    __shared__ unsigned long long hits[DIRECT_WORDS];
+    __shared__ uint32_t idx[ROUND], scan_lds[4], list_base;
+    if (uniform(b.cnt->overflow) != 0) return;
+    const uint32_t nft = uniform(b.head->nftiles), ns = uniform(b.head->nscenes);
+    const uint32_t t = threadIdx.x, wave = uniform(t >> 6), lane = t & 63u;
+    // the coarse entries the job would have had (a count callers can read),
+    // from k_setup's per-wave counts: few workgroups add to one counter
+    constexpr uint32_t ADDERS = 32;
+    if (blockIdx.x < ADDERS) {
+        const uint32_t n = b.head->ntri / 64u, step = min(gridDim.x, ADDERS) * 256u;
+        uint32_t pairs = 0, all;
+        for (uint32_t i = blockIdx.x * 256u + t; i < n; i += step) pairs += b.wave_prims[i];
+        (void)block_exclusive_scan<uint32_t>(pairs, scan_lds, &all);
+        if (t == 0 && all != 0) atomicAdd(&b.cnt->pairs_binned, all);
+    }
+    for (uint32_t ft = blockIdx.x; ft < nft; ft += gridDim.x) {
+        const uint32_t s = find_scene_ftile(scenes, ns, ft);
+        const SceneCfg& sc = scenes[s];
+        const uint32_t W = sc.W, H = sc.H;
+        const uint32_t nfx = (W + 31u) / 32u, at = ft - sc.ftile_base;
+        const uint32_t fx = at % nfx, fy = at / nfx, ox = fx * 32u, oy = fy * 32u;
+        const uint32_t P = min(runs[s].nprims, DIRECT_WORDS * 64u), words = (P + 63u) / 64u;
+        const uint4* pb = pbin + runs[s].prim_base;
+        constexpr uint32_t AHEAD = 4;
+        for (uint32_t w0 = wave; w0 < words; w0 += 4u * AHEAD) {
+            uint4 v[AHEAD];
+#pragma unroll
+            for (uint32_t k = 0; k < AHEAD; ++k) v[k] = pb[min((w0 + 4u * k) * 64u + lane, P - 1u)];
+#pragma unroll
+            for (uint32_t k = 0; k < AHEAD; ++k) {
+                const uint32_t w = w0 + 4u * k, i = w * 64u + lane;
+                const uint32_t x0 = v[k].y & 0xFFFFu, x1 = v[k].y >> 16, y0 = v[k].z & 0xFFFFu, y1 = v[k].z >> 16;
+                const bool hit = (i < P) & (x0 < x1) & (y0 < y1) & (x0 < ox + 32u) & (x1 > ox) & (y0 < oy + 32u) & (y1 > oy);
+                const uint64_t m = ballot(hit);
+                if (w < words && lane == 0) hits[w] = m;
+            }
+        }
+        __syncthreads();
+        // thread t's words, in order: their hits, and the hits before them
+        const uint32_t per = (words + 255u) / 256u, wb = min(t * per, words), we = min(wb + per, words);
+        uint32_t own = 0, total;
+        for (uint32_t w = wb; w < we; ++w) own += (uint32_t)__popcll(hits[w]);
+        const uint32_t before = block_exclusive_scan<uint32_t>(own, scan_lds, &total);
+        if (t == 0) list_base = total != 0 ? atomicAdd(&b.cnt->fine_total, total) : 0u;
+        __syncthreads();
+        const uint32_t base = list_base;
+        const bool fits = base <= b.fine_cap && total <= b.fine_cap - base;
+        if (!fits) {
+            if (t == 0) atomicOr(&b.cnt->overflow, OVF_FINE);
+        } else {
+            // the set bits' indices go to LDS at their positions, then a thread
+            // each loads, makes and stores the entries (bit by bit, a word's
+            // loads would wait for one another)
+            for (uint32_t lo = 0; lo < total; lo += ROUND) {
+                uint32_t pos = before - lo;  // (below 0 wraps past ROUND)
+                for (uint32_t w = wb; w < we; ++w)
+                    for (unsigned long long m = hits[w]; m != 0; m &= m - 1, ++pos)
+                        if (pos < ROUND) idx[pos] = w * 64u + (uint32_t)__builtin_ctzll(m);
+                __syncthreads();
+                const uint32_t n = min(total - lo, ROUND);
+                for (uint32_t k = t; k < n; k += 256u) {
+                    const uint4 e = pb[idx[k]];
+                    const uint32_t qm = fine_quad_bits(5u, e.y & 0xFFFFu, e.y >> 16, e.z & 0xFFFFu, e.z >> 16, ox, oy);
+                    b.flist[base + lo + k] = make_uint2(runs[s].prim_base + idx[k], zlo_key(e.w, 16u) | qm);
+                }
+                __syncthreads();
+            }
+            // the records of the tile's four raster tiles' quadrants
+            const uint32_t tx = fx * 2u + ((t >> 2) & 1u), ty = fy * 2u + ((t >> 3) & 1u), q = t & 3u;
+            const uint32_t ntx = (W + 15u) / 16u, nty = (H + 15u) / 16u;
+            if (t < 16u && tx < ntx && ty < nty) {
+                const uint32_t slot = sc.raster_base + blocked_rank(tx, ty, ntx, nty);
+                if (slot < b.tile_cap)
+                    b.tile_rec[4u * slot + q] = make_uint4(s, base, base + total, (tx * 16u + (q & 1u) * 8u) |
+                                                                                      (ty * 16u + (q >> 1) * 8u) << 16);
+            }
+        }
+        __syncthreads();  // hits, scan_lds and list_base are the next tile's
     }
 }
 
@@ -2762,25 +2887,29 @@ void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_s
     k_setup<<<at_least1(g.tris), 256, 0, s>>>(b, b.draws, b.scenes, b.runs, b.tchunk_draw, b.chunk_off, b.nsub, b.cls,
                                               b.clip_out);
     if (ev_bin) (void)hipEventRecord(ev_bin, s);
-    k_bin<false><<<at_least1(g.bins), 256, 0, s>>>(b, b.pchunk_scene, b.scenes, b.runs, b.pbin, b.bin_offsets);
-    launch_scan<uint32_t>(s, b.bin_counts, b.bin_offsets, b.mat_cap, &b.cnt->mat_len, b.parts,
-                          &b.cnt->pairs_binned);
-    k_bin<true><<<at_least1(g.bins), 256, 0, s>>>(b, b.pchunk_scene, b.scenes, b.runs, b.pbin, b.bin_offsets);
-    // fine_chunks and fmat_len are adjacent: the u64 total fills both
-    if (b.bins_cap <= FINE_PREP_ONE_MAX) {
-        k_fine_prep_one<<<1, 256, 0, s>>>(b);
+    if (g.direct != 0) {
+        k_tile_bin<<<g.direct, 256, 0, s>>>(b, b.pbin, b.scenes, b.runs);
     } else {
-        k_fine_prep<<<at_least1(std::min<uint32_t>((b.bins_cap + 255) / 256, 1024u)), 256, 0, s>>>(b);
-        launch_scan<unsigned long long>(s, b.fpack, b.fpre, b.bins_cap, &b.head->nbins, b.parts64,
-                                        reinterpret_cast<unsigned long long*>(&b.cnt->fine_chunks));
-        k_fchunk_map<<<at_least1(std::min<uint32_t>((b.bins_cap + 255) / 256, 1024u)), 256, 0, s>>>(b);
+        k_bin<false><<<at_least1(g.bins), 256, 0, s>>>(b, b.pchunk_scene, b.scenes, b.runs, b.pbin, b.bin_offsets);
+        launch_scan<uint32_t>(s, b.bin_counts, b.bin_offsets, b.mat_cap, &b.cnt->mat_len, b.parts,
+                              &b.cnt->pairs_binned);
+        k_bin<true><<<at_least1(g.bins), 256, 0, s>>>(b, b.pchunk_scene, b.scenes, b.runs, b.pbin, b.bin_offsets);
+        // fine_chunks and fmat_len are adjacent: the u64 total fills both
+        if (b.bins_cap <= FINE_PREP_ONE_MAX) {
+            k_fine_prep_one<<<1, 256, 0, s>>>(b);
+        } else {
+            k_fine_prep<<<at_least1(std::min<uint32_t>((b.bins_cap + 255) / 256, 1024u)), 256, 0, s>>>(b);
+            launch_scan<unsigned long long>(s, b.fpack, b.fpre, b.bins_cap, &b.head->nbins, b.parts64,
+                                            reinterpret_cast<unsigned long long*>(&b.cnt->fine_chunks));
+            k_fchunk_map<<<at_least1(std::min<uint32_t>((b.bins_cap + 255) / 256, 1024u)), 256, 0, s>>>(b);
+        }
+        k_fine_bin<false><<<at_least1(g.fine), 256, 0, s>>>(b, b.fchunk_rec, b.scenes, b.fpre, b.bin_rng, b.list,
+                                                     b.fine_off);
+        launch_scan<uint32_t>(s, b.fine_counts, b.fine_off, b.fmat_cap, &b.cnt->fmat_len, b.parts, &b.cnt->fine_total);
+        k_fine_bin<true><<<at_least1(g.fine), 256, 0, s>>>(b, b.fchunk_rec, b.scenes, b.fpre, b.bin_rng, b.list,
+                                                    b.fine_off);
+        k_tile_prep<<<at_least1(std::min<uint32_t>((4u * g.ntiles + 255) / 256, 4096u)), 256, 0, s>>>(b);
     }
-    k_fine_bin<false><<<at_least1(g.fine), 256, 0, s>>>(b, b.fchunk_rec, b.scenes, b.fpre, b.bin_rng, b.list,
-                                                 b.fine_off);
-    launch_scan<uint32_t>(s, b.fine_counts, b.fine_off, b.fmat_cap, &b.cnt->fmat_len, b.parts, &b.cnt->fine_total);
-    k_fine_bin<true><<<at_least1(g.fine), 256, 0, s>>>(b, b.fchunk_rec, b.scenes, b.fpre, b.bin_rng, b.list,
-                                                b.fine_off);
-    k_tile_prep<<<at_least1(std::min<uint32_t>((4u * g.ntiles + 255) / 256, 4096u)), 256, 0, s>>>(b);
     if (ev_raster) (void)hipEventRecord(ev_raster, s);
     if (svc) {
         k_svc_post<<<1, 64, 0, s>>>(b, svc, svc_host, svc_ctl, svc_index);
