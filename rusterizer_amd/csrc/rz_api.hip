@@ -167,7 +167,7 @@ struct rz_ctx {
     FrameCounters* h_cnt = nullptr;  // pinned
 
     // pipeline buffers
-    DBuf<uint32_t> cls, nsub, wave_prims, chunk_off, parts;
+    DBuf<uint32_t> cls, nsub, wave_prims, wave_pairs, chunk_off, parts;
     DBuf<unsigned long long> parts64;
     DBuf<uint32_t> clip_tri, clip_draw;
     DBuf<float> clip_out;  // MAXV * 10 floats per slot
@@ -191,9 +191,10 @@ struct rz_ctx {
     DBuf<float> msaa_depth;
     uint64_t gen = 0;  // bumped whenever a buffer moves (invalidates the graph)
 
-    // graphs of the launch sequence: with coarse and fine binning, and with
-    // k_tile_bin (a context that serves jobs of both kinds keeps both)
-    JobGraph graphs[2];
+    // graphs of the launch sequence: with coarse and fine binning, with
+    // k_tile_bin, and that without k_scene_prep (a context that serves jobs of
+    // several kinds keeps them all)
+    JobGraph graphs[3];
     uint32_t tiles_cap = 0;  // raster grid of the graphs: most tiles of any job so far
 
     hipEvent_t done = nullptr;
@@ -501,12 +502,16 @@ int size_buffers(rz_ctx* c, const JobPlan& pl, const Needs& n_in, G& g) {
     n.clip = std::max<uint64_t>(n.clip, NT / 8 + 1024);
     n.pairs = std::max<uint64_t>(n.pairs, n.prims * 2);
     n.fine = std::max<uint64_t>(n.fine, std::max<uint64_t>(c->flist.cap, n.pairs * 8));
+    // lists placed without reservation (k_tile_bin), up to 16 MB of them
+    if (pl.direct && pl.nscenes == 1)
+        n.fine = std::max<uint64_t>(n.fine, std::min<uint64_t>((uint64_t)pl.nftiles * (NT + NT / 4), 2ull << 20));
     const uint64_t lim = 0xF0000000ull;
     if (n.prims > lim || n.pairs > lim || n.fine > lim || n.clip > lim)
         return fail(c, RZ_ERR_LIMIT, "job needs more than 2^32 pipeline entries");
     const size_t cls = g(c->cls, std::max<uint64_t>(NT, 256));
     g(c->nsub, cls);
     g(c->wave_prims, cls / 64 + 4);
+    if (pl.direct) g(c->wave_pairs, cls / 64 + 4);
     g(c->chunk_off, cls / TRI_ALIGN + 1);
     const size_t geom = g(c->geom, n.prims);
     g(c->attrs, geom * ATTR_STRIDE);
@@ -606,7 +611,7 @@ uint64_t held(const DBuf<T>& b) {
 
 // device bytes of the context's pipeline buffers, outputs and tables
 uint64_t ctx_bytes(const rz_ctx* c) {
-    uint64_t n = held(c->cls) + held(c->nsub) + held(c->wave_prims) + held(c->chunk_off) + held(c->parts) + held(c->parts64) +
+    uint64_t n = held(c->cls) + held(c->nsub) + held(c->wave_prims) + held(c->wave_pairs) + held(c->chunk_off) + held(c->parts) + held(c->parts64) +
                  held(c->clip_tri) + held(c->clip_draw) + held(c->clip_out) + held(c->geom) +
                  held(c->attrs) + held(c->uvat) + held(c->pbin) + held(c->bin_counts) + held(c->bin_offsets) + held(c->list) +
                  held(c->bin_rng) + held(c->tile_rec) + held(c->fchunk_rec) + held(c->tchunk_draw) +
@@ -620,6 +625,9 @@ uint64_t ctx_bytes(const rz_ctx* c) {
 }
 
 uint32_t init_split(uint32_t draws);
+
+// k_setup does without k_scene_prep
+bool one_scene(const JobPlan& pl) { return pl.direct && pl.nscenes == 1 && pl.ntri <= DIRECT_TRIS; }
 
 JobBufs job_bufs(const rz_ctx* c) {
     JobBufs b{};
@@ -642,6 +650,7 @@ JobBufs job_bufs(const rz_ctx* c) {
     b.cls = c->cls.p;
     b.nsub = c->nsub.p;
     b.wave_prims = c->wave_prims.p;
+    b.wave_pairs = c->wave_pairs.p;
     b.chunk_off = c->chunk_off.p;
     b.clip_tri = c->clip_tri.p;
     b.clip_draw = c->clip_draw.p;
@@ -682,6 +691,7 @@ JobBufs job_bufs(const rz_ctx* c) {
     b.clip_wide = c->clip_wide ? 1u : 0u;
     b.exact_paths = c->exact_paths ? 1u : 0u;
     b.direct = c->plan.direct ? 1u : 0u;
+    b.one_scene = one_scene(c->plan) ? 1u : 0u;
     return b;
 }
 
@@ -819,7 +829,7 @@ int enqueue_graph(rz_ctx* c, const JobPlan& pl) {
     const int svc = c->job_svc ? c->svc_entry : -1;
     if (pl.ntiles > c->tiles_cap) c->tiles_cap = std::max<uint32_t>(pl.ntiles, c->tiles_cap + c->tiles_cap / 4);
     const JobGrid g = job_grid(c, pl, true);
-    JobGraph& jg = c->graphs[pl.direct ? 1 : 0];
+    JobGraph& jg = c->graphs[one_scene(pl) ? 2 : pl.direct ? 1 : 0];
     if (!jg.exec || jg.gen != c->gen || jg.dcap != c->dcap || jg.scap != c->scap || jg.raster != g.raster ||
         jg.tiles != g.ntiles || jg.stats != c->raster_stats || jg.svc != svc) {
         if (jg.exec) {
@@ -1466,6 +1476,7 @@ int rz_destroy(rz_ctx* c) {
     release(c->cls);
     release(c->nsub);
     release(c->wave_prims);
+    release(c->wave_pairs);
     release(c->chunk_off);
     release(c->parts);
     release(c->parts64);
@@ -1687,6 +1698,7 @@ int rz_trim(rz_ctx* c) {
     release(c->cls);
     release(c->nsub);
     release(c->wave_prims);
+    release(c->wave_pairs);
     release(c->chunk_off);
     release(c->parts);
     release(c->parts64);

@@ -161,8 +161,8 @@ struct JobBufs {
     // geometry
     uint32_t* cls;
     uint32_t* nsub;       // rasterizer triangles of each clipped triangle
-    uint32_t* wave_prims; // rasterizer triangles of each 64 triangles; with direct, k_setup leaves its
-                          // waves' coarse entries here
+    uint32_t* wave_prims; // rasterizer triangles of each 64 triangles
+    uint32_t* wave_pairs; // with direct: coarse entries of each of k_setup's waves
     uint32_t* chunk_off;  // per TRI_ALIGN-triangle chunk: the rasterizer triangles of all earlier ones
     uint32_t* clip_tri;   // clipped triangle of each clip slot
     uint32_t* clip_draw;  // its draw
@@ -196,6 +196,7 @@ struct JobBufs {
     uint32_t tchunk_cap, pchunk_cap, rstat_cap;  // rstat_cap in workgroups
     uint32_t clip_wide;    // clip every polygon with a full wave
     uint32_t direct;       // binned by k_tile_bin
+    uint32_t one_scene;    // k_setup does k_scene_prep's work (one scene of at most DIRECT_TRIS padded triangles)
     uint32_t exact_paths;  // setup proves nothing: every prim takes the raster's exact paths
     uint32_t* svc_flags;   // raster service: pinned host array of the scenes' final flags
     // the job tables as the host wrote them (pinned host memory, or the

@@ -306,9 +306,12 @@ struct ClipV {
 };
 
 // Returns true in the lanes of a group whose polygon needs more than G lanes
-// (nothing is written for it then).
+// (nothing is written for it then); tri: the triangle, prims: its rasterizer
+// triangles (the same in every lane of the group).
 template <uint32_t G>
-__device__ __forceinline__ bool clip_polygon(const JobBufs& b, uint32_t slot, bool have, float* __restrict__ sh) {
+__device__ __forceinline__ bool clip_polygon(const JobBufs& b, uint32_t slot, bool have, float* __restrict__ sh,
+                                             uint32_t& tri, uint32_t& prims) {
+    tri = prims = 0;
     const uint32_t lane = threadIdx.x & 63u, gl = lane & (G - 1), gb = lane - gl;
     const uint64_t gmask = G == 64 ? ~0ull : (((1ull << G) - 1) << gb);
     float* q = sh + gb * 10;  // this group's staging area: G vertices
@@ -317,7 +320,7 @@ __device__ __forceinline__ bool clip_polygon(const JobBufs& b, uint32_t slot, bo
     v.x = v.y = v.z = v.w = 0.0f;
     for (int j = 0; j < 6; ++j) v.a[j] = 0.0f;
     if (have) {
-        t = b.clip_tri[slot];
+        t = tri = b.clip_tri[slot];
         const uint32_t d = b.clip_draw[slot];
         const DrawDev& dd = b.draws[d];
         scene = dd.scene;
@@ -413,10 +416,8 @@ __device__ __forceinline__ bool clip_polygon(const JobBufs& b, uint32_t slot, bo
     } else if (n > 0) {
         if (gl == 0) atomicOr(&b.runs[scene].flags, RZ_FLAG_CLIP_FEWER);
     }
-    if (gl == 0) {
-        b.nsub[t] = ntris;
-        if (ntris != 0) atomicAdd(&b.wave_prims[t / 64u], ntris);
-    }
+    if (gl == 0) b.nsub[t] = ntris;
+    prims = ntris;
     return false;
 }
 
@@ -426,20 +427,37 @@ __device__ __forceinline__ bool clip_polygon(const JobBufs& b, uint32_t slot, bo
 __global__ __launch_bounds__(64) void k_clip(JobBufs b) {
     __shared__ float sh[64 * 10];
     const uint32_t nslots = min(uniform(b.cnt->nclip), b.clip_cap);
+    uint32_t tri, prims;
+    auto whole_wave = [&](uint32_t slot) {
+        (void)clip_polygon<64>(b, slot, true, sh, tri, prims);
+        if (threadIdx.x == 0 && prims != 0) atomicAdd(&b.wave_prims[tri / 64u], prims);
+    };
     if (b.clip_wide) {
-        for (uint32_t i = blockIdx.x; i < nslots; i += gridDim.x) (void)clip_polygon<64>(b, i, true, sh);
+        for (uint32_t i = blockIdx.x; i < nslots; i += gridDim.x) whole_wave(i);
         return;
     }
     constexpr uint32_t G = 64 / CLIP_GROUPS;
     for (uint32_t base = blockIdx.x * CLIP_GROUPS; base < nslots; base += gridDim.x * CLIP_GROUPS) {
         const uint32_t slot = base + threadIdx.x / G;
-        const bool big = clip_polygon<G>(b, slot, slot < nslots, sh);
+        const bool big = clip_polygon<G>(b, slot, slot < nslots, sh, tri, prims);
+        // the counts go to the triangles' groups of 64, one atomic per group of
+        // the wave's polygons (in triangle order, so mostly one or two groups; an
+        // atomic each cost the 4M-triangle terrain's clipping 20 of 60 us)
+        const uint32_t key = tri / 64u;
+        uint32_t sum = 0;
+        bool first = true;
+        for (uint32_t h = 0; h < CLIP_GROUPS; ++h) {
+            const bool same = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)(h * G)) == key;
+            sum += same ? (uint32_t)__builtin_amdgcn_readlane((int)prims, (int)(h * G)) : 0u;
+            first = first && !(same && h < threadIdx.x / G);
+        }
+        if (threadIdx.x % G == 0 && first && sum != 0) atomicAdd(&b.wave_prims[key], sum);
         // one bit per group whose polygon was too big: lane G * k of group k
         uint64_t redo = __ballot(big && (threadIdx.x % G) == 0);
         while (redo != 0) {
             const uint32_t k = (uint32_t)__ffsll((unsigned long long)redo) - 1u;
             redo &= redo - 1;
-            (void)clip_polygon<64>(b, base + k / G, true, sh);
+            whole_wave(base + k / G);
         }
     }
 }
@@ -889,9 +907,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     __shared__ PrimGeom stage[SETUP_STAGE];
     __shared__ uint32_t poff[256], pcls[256];  // per triangle of the chunk: first prim (chunk-relative), class
     __shared__ uint32_t wtot[4];               // per wave of the chunk: its prims
+    __shared__ uint32_t woff[256];             // one scene: prims before each wave's triangles
     if (uniform(b.cnt->overflow) != 0) return;
     const uint32_t NT = b.head->ntri;
     const uint32_t prim_cap = b.prim_cap;
+    const bool one = b.one_scene != 0;
+    if (one) {
+        // k_scene_prep's work for a single small scene, by every workgroup for
+        // itself: 64 chunks of four waves are one count a thread, where the
+        // launch of its own took 8 us of an 80 us frame
+        uint32_t total;
+        const uint32_t before = block_exclusive_scan<uint32_t>(
+            threadIdx.x < NT / 64u ? b.wave_prims[threadIdx.x] : 0u, wtot, &total);
+        woff[threadIdx.x] = before;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            const uint32_t nch = (total + CHUNK - 1u) / CHUNK;
+            SceneRun& r = b.runs[0];
+            r.prim_off = 0;
+            r.nprims = total;
+            r.prim_base = 0;
+            r.chunk_base = 0;
+            r.nch = nch;
+            r.mat_base = 0;
+            b.cnt->nprims_raw = total;
+            b.cnt->nchunks = nch;
+            b.cnt->nprims = nch * CHUNK;
+            if (nch * CHUNK > prim_cap) atomicOr(&b.cnt->overflow, OVF_PRIMS);
+        }
+        __syncthreads();
+    }
     // the chunk table words of the workgroup's next chunk are loaded one
     // chunk ahead (NT is a multiple of 256)
     uint32_t n_d = 0, n_s0 = 0, n_sub = 0, n_cls = 0;
@@ -899,7 +943,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         if (c * 256u < NT) {
             const uint32_t c0 = c * 256u;
             n_d = tchunk_draw[c];
-            n_s0 = chunk_off[c];
+            n_s0 = one ? woff[c * 4u] : chunk_off[c];
             n_sub = nsub[c0 + threadIdx.x];
             n_cls = cls[c0 + threadIdx.x];
         }
@@ -920,7 +964,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         const bool tex_idx32 = dd.tw < (1u << 24) && dd.th < (1u << 24) && (uint64_t)dd.tw * dd.th <= 0xFFFFFFFFull;
         const bool proofs = b.exact_paths == 0;
         // the chunk's prim range (its 256 triangles belong to draw d: draws are 256-aligned)
-        const uint32_t blk_first = uniform(run.prim_base + (s0 - run.prim_off));
+        const uint32_t blk_first = one ? s0 : uniform(run.prim_base + (s0 - run.prim_off));
         // each triangle's first prim: prefix sum of the counts (below 16: four
         // bit planes) over the wave, then over the waves
         uint32_t pre = 0, mine = 0;
@@ -988,7 +1032,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         }
         if (per_bin != 0) {
             for (int o = 32; o >= 1; o >>= 1) pairs += (uint32_t)__shfl_xor((int)pairs, o);
-            if (lane_id() == 0) b.wave_prims[blk * 4u + wave] = pairs;
+            if (lane_id() == 0) b.wave_pairs[blk * 4u + wave] = pairs;
         }
         __syncthreads();
         if (staged) {
@@ -1440,7 +1484,7 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
     if (blockIdx.x < ADDERS) {
         const uint32_t n = b.head->ntri / 64u, step = min(gridDim.x, ADDERS) * 256u;
         uint32_t pairs = 0, all;
-        for (uint32_t i = blockIdx.x * 256u + t; i < n; i += step) pairs += b.wave_prims[i];
+        for (uint32_t i = blockIdx.x * 256u + t; i < n; i += step) pairs += b.wave_pairs[i];
         (void)block_exclusive_scan<uint32_t>(pairs, scan_lds, &all);
         if (t == 0 && all != 0) atomicAdd(&b.cnt->pairs_binned, all);
     }
@@ -1472,7 +1516,10 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
         uint32_t own = 0, total;
         for (uint32_t w = wb; w < we; ++w) own += (uint32_t)__popcll(hits[w]);
         const uint32_t before = block_exclusive_scan<uint32_t>(own, scan_lds, &total);
-        if (t == 0) list_base = total != 0 ? atomicAdd(&b.cnt->fine_total, total) : 0u;
+        // one scene whose tiles' longest possible lists fit side by side needs
+        // no reservation (an atomic on one counter is 7 ns a tile and 2 us late)
+        const bool placed = ns == 1u && (uint64_t)nft * P <= b.fine_cap;
+        if (t == 0) list_base = placed ? ft * P : total != 0 ? atomicAdd(&b.cnt->fine_total, total) : 0u;
         __syncthreads();
         const uint32_t base = list_base;
         const bool fits = base <= b.fine_cap && total <= b.fine_cap - base;
@@ -2883,7 +2930,7 @@ void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_s
     k_job_init<<<at_least1(g.init), 256, 0, s>>>(b);
     k_classify<<<at_least1(std::min<uint32_t>(g.tris, 2048u)), 256, 0, s>>>(b, b.tchunk_draw, b.draws);
     k_clip<<<at_least1((g.clip + CLIP_GROUPS - 1) / CLIP_GROUPS), 64, 0, s>>>(b);
-    k_scene_prep<<<1, 1024, 0, s>>>(b);
+    if (!b.one_scene) k_scene_prep<<<1, 1024, 0, s>>>(b);
     k_setup<<<at_least1(g.tris), 256, 0, s>>>(b, b.draws, b.scenes, b.runs, b.tchunk_draw, b.chunk_off, b.nsub, b.cls,
                                               b.clip_out);
     if (ev_bin) (void)hipEventRecord(ev_bin, s);

@@ -75,3 +75,14 @@ def test_tile_bin_batches_switch_between_the_binnings():
                 assert_parity(g, want[id(sc)], where=sc.name)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("draws", [0, 64, 65])
+def test_tile_bin_frames_of_many_draws(draws):
+    """Each draw starts a chunk of 256 triangles of its own: 64 chunks are the
+    most a frame's k_setup workgroups add up by themselves."""
+    parts = [_frame(3 + i % 5, 90, 50, 25, seed=100 + i) for i in range(draws)]
+    if not parts:
+        parts = [_frame(1, 90, 50, 25, seed=1)]
+        parts[0].idx = parts[0].idx[:0]
+    assert_parity(run_gpu(parts), run_oracle(parts), where=f"{draws} draws")
