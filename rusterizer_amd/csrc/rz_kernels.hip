@@ -700,9 +700,13 @@ __global__ __launch_bounds__(1024) void k_scene_prep(JobBufs b) {
 // ---------------------------------------------------------------------------
 // The raster's matrix path (walk_rows): tolerance of its values, and the largest
 // distance of a depth it stores from the reference's (half the tolerance: two
-// stored depths are compared). WALK_EZ = 32u: the plane's own error at depths
-// up to 1 is 18u (depth_plane_bound).
-constexpr float WALK_TOL = 0x1p-18f, WALK_EZ = 0x1p-19f;
+// stored depths are compared). WALK_EZ = 128u: the plane's own error is 18u at
+// depths up to 1 and grows with its rise over the prim's quadrants
+// (depth_plane_bound). A smaller value sends the steep prims of the near plane
+// down the exact path, a larger one more pairs of close depths: raster of 256
+// textured scenes at 32u, 64u, 128u, 256u, 512u: 5.50, 5.23, 5.13, 5.13, 5.17 ms;
+// 1M-triangle soup 0.370, 0.355, 0.346, 0.348, 0.350 ms.
+constexpr float WALK_TOL = 0x1p-16f, WALK_EZ = 0x1p-17f;
 constexpr uint32_t NO_SCALE = 0x7FC00000u;  // a NaN: no margin known
 
 __device__ __forceinline__ bool tie_rule(float nx, float ny) {
@@ -1874,10 +1878,10 @@ static_assert(offsetof(PrimGeom, nx0) == 24 && offsetof(PrimGeom, pzx) == 48 && 
 // path are within WALK_EZ of the reference's; where one's exact value matters it
 // is computed again from the sample's winner.
 // The walk is bound by instruction issue: a prim takes 35 vector instructions
-// here against about 120 by the reference's steps, and about 1.2% of the prims
-// fall in the margins (2.2% of a deep 1080p soup's). Raster of 256 textured
-// scenes 6.55 -> 5.41 ms, of a 1M-triangle 1080p soup 0.419 -> 0.366 ms, of a
-// 4M-triangle 4K terrain 0.348 -> 0.217 ms. Groups of 8 prims against 4: the
+// here against about 120 by the reference's steps; 4 to 6% of the prims take
+// those. Raster of 256 textured
+// scenes 6.55 -> 5.13 ms, of a 1M-triangle 1080p soup 0.419 -> 0.346 ms, of a
+// 4M-triangle 4K terrain 0.348 -> 0.220 ms. Groups of 8 prims against 4: the
 // terrain's 0.217 against 0.234 ms, the batch the same.
 typedef float MfmaAcc __attribute__((ext_vector_type(16)));
 typedef __bf16 MfmaIn __attribute__((ext_vector_type(8)));

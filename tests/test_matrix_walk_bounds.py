@@ -17,7 +17,7 @@ from tests.test_cull_bounds import RGSS, clamp01, covered_depths, setup
 
 F = np.float32
 U = 2.0 ** -24
-TOL, EZ = 2.0 ** -18, 2.0 ** -19
+TOL, EZ = 2.0 ** -16, 2.0 ** -17
 
 
 def fma(a, b, c):
