@@ -1684,11 +1684,9 @@ __device__ __forceinline__ float edge(float nx, float ny, float ax, float ay, fl
     return nx * (x - ax) + ny * (y - ay);
 }
 
-// an edge function's largest value on the square of half side 3.875 px about
-// (xc, yc), with FMA (used against a margin only)
-__device__ __forceinline__ float corner_edge(float nx, float ny, float ax, float ay, float xc, float yc) {
-    const float c = __builtin_fmaf(ny, yc - ay, nx * (xc - ax));
-    return __builtin_fmaf(3.875f, fabsf(nx) + fabsf(ny), c);
+// an edge function's value at (xc, yc), with FMA (used against margins only)
+__device__ __forceinline__ float centre_edge(float nx, float ny, float ax, float ay, float xc, float yc) {
+    return __builtin_fmaf(ny, yc - ay, nx * (xc - ax));
 }
 
 // bits 0..3 of v as bytes 0x00 or 0xFF
@@ -1867,7 +1865,7 @@ static_assert(offsetof(PrimGeom, nx0) == 24 && offsetof(PrimGeom, pzx) == 48 && 
 // values and its depth at all 256 samples of a quadrant: row (k, h, f) of the
 // left matrix is function f (edges 0-2, depth) at sample k of pixel row half
 // h, as coefficients of (X, Y, 1); column c of the right one is pixel (c & 7,
-// c >> 3) of a half, in eighths of a pixel (exact in bf16). Each coefficient is
+// c >> 3) of a half, in eighths of a pixel from its centre (exact in bf16). Each coefficient is
 // split into three bf16 parts that add up to it exactly, so the products are
 // exact and only their f32 sum rounds. Lane l of the result holds the four
 // functions of its own pixel's four samples. The edge functions are scaled
@@ -1878,10 +1876,12 @@ static_assert(offsetof(PrimGeom, nx0) == 24 && offsetof(PrimGeom, pzx) == 48 && 
 // path are within WALK_EZ of the reference's; where one's exact value matters it
 // is computed again from the sample's winner.
 // The walk is bound by instruction issue: a prim takes 35 vector instructions
-// here against about 120 by the reference's steps; 4 to 6% of the prims take
-// those. Raster of 256 textured
-// scenes 6.55 -> 5.13 ms, of a 1M-triangle 1080p soup 0.419 -> 0.346 ms, of a
-// 4M-triangle 4K terrain 0.348 -> 0.220 ms. Groups of 8 prims against 4: the
+// here against about 120 by the reference's steps; 2 to 13% of the prims take
+// those, and look up an exact stored depth only for samples where it decides.
+// Raster of 256 textured scenes 6.55 -> 5.00 ms (5.21 with every stored depth
+// made exact for each such prim and the records loaded again for the rows), of
+// a 1M-triangle 1080p soup 0.419 -> 0.341 ms, of a 4M-triangle 4K terrain
+// 0.348 -> 0.220 ms. Groups of 8 prims against 4: the
 // terrain's 0.217 against 0.234 ms, the batch the same.
 typedef float MfmaAcc __attribute__((ext_vector_type(16)));
 typedef __bf16 MfmaIn __attribute__((ext_vector_type(8)));
@@ -1895,14 +1895,23 @@ struct alignas(16) WalkRows {
 };
 static_assert(sizeof(WalkRows) == 320, "WalkRows layout");
 
-// LDS of one wave's walk: the candidate queue (at most QUEUE_RUN + 63
-// entries) and the rows of a group of prims
-constexpr uint32_t WAVE_QUEUE = 112;
+// a candidate's three scaled edge functions and depth plane about the centre
+// of its quadrant: component f is function f
+struct WalkCoef {
+    float4 a, b, c;  // per eighth of a pixel in x and y, at the centre
+};
+
+// LDS of one wave's walk: the candidate queue (at most walk_batch + 63
+// entries), the coefficients of a batch and the rows of a group of prims. The
+// batch is what 32 waves of a CU have room for beside the rows: 5 KB a wave.
+constexpr uint32_t walk_batch(uint32_t waves) { return waves == 1 ? 44u : 24u; }
 template <uint32_t R>
 struct alignas(16) WalkLds {
-    uint32_t queue[WAVE_QUEUE];
+    WalkCoef coef[walk_batch(R)];
     WalkRows rows[walk_group(R)];
+    uint32_t queue[(walk_batch(R) + 63u + 3u) / 4u * 4u];
 };
+static_assert(sizeof(WalkLds<1>) <= 5120, "eight waves per SIMD");
 
 // LDS of the raster: per wave (R waves) the walk's working space, then in the
 // shading stage its tasks {prim, owner lane | pass mask << 6}, their colours,
@@ -1967,24 +1976,18 @@ __device__ __forceinline__ uint32_t hi16_pair(float lo, float hi) {  // top halv
 }
 __device__ __forceinline__ float top8(float x) { return __uint_as_float(__float_as_uint(x) & 0xFFFF0000u); }
 
-// Writes the rows of a group of prims for the quadrant at (qx0, qy0). Lane 8p
-// + 4h + f takes function f for row half h of the group's prim p (the lane's
-// own argument; any record will do past the group's last). Samples 0 and 2 lie
-// at +-(1, -3) eighths of a pixel from the pixel's centre, 1 and 3 at +-(3, 1).
-__device__ __forceinline__ void walk_rows(const PrimGeom* __restrict__ geom, uint32_t prim, WalkRows* rows, uint32_t lane,
-                                          float cx8, float cy8) {
+// Writes the rows of a group of prims from their coefficients. Lane 8p + 4h +
+// f takes function f for row half h of the group's prim p, candidate k of the
+// batch (the lane's own argument; any will do past the group's last). Samples 0
+// and 2 lie at +-(1, -3) eighths of a pixel from the pixel's centre, 1 and 3 at
+// +-(3, 1).
+__device__ __forceinline__ void walk_rows(const WalkCoef* coef, uint32_t k, WalkRows* rows, uint32_t lane) {
     const uint32_t f = lane & 3u;
-    const float* rec = reinterpret_cast<const float*>(geom + prim);
-    const float2 n = *reinterpret_cast<const float2*>(rec + 6 + 2 * f);  // the depth's slopes follow the normals
-    const float2 a = *reinterpret_cast<const float2*>(rec + 2 * min(f, 2u));
-    const float rs = rec[14], z2 = rec[19];
-    const bool isz = f == 3u;
-    const float sc = isz ? 0.125f : rs * 0.125f;
-    const float A = n.x * sc, B = n.y * sc;  // per eighth of a pixel
-    // the value at the centre of the half's first pixel
-    const float dx = __builtin_fmaf(-8.0f, a.x, cx8), dy = __builtin_fmaf(-8.0f, a.y, cy8);
-    const float c0 = __builtin_fmaf(A, dx, __builtin_fmaf(B, dy, isz ? z2 : 0.0f));
-    const float c = __builtin_fmaf((lane & 4u) ? 32.0f : 0.0f, B, c0);
+    const float* const cf = reinterpret_cast<const float*>(reinterpret_cast<const char*>(coef) +
+                                                           __umul24(k, (uint32_t)sizeof(WalkCoef))) + f;
+    const float A = cf[0], B = cf[4];
+    // at the centre of the half
+    const float c = __builtin_fmaf((lane & 4u) ? 16.0f : -16.0f, B, cf[8]);
     const float p = __builtin_fmaf(-3.0f, B, A), q = __builtin_fmaf(3.0f, A, B);
     const float A2 = A - top8(A), B2 = B - top8(B);
     char* const r = reinterpret_cast<char*>(rows) + __umul24(lane >> 3, (uint32_t)sizeof(WalkRows));
@@ -1992,9 +1995,9 @@ __device__ __forceinline__ void walk_rows(const PrimGeom* __restrict__ geom, uin
     *reinterpret_cast<uint4*>(r + offsetof(WalkRows, ab) + 16u * f) =
         make_uint4(hi16_pair(A, A2), hi16_pair(A2 - top8(A2), B), hi16_pair(B2, B2 - top8(B2)), 0u);
     uint2* const rc = reinterpret_cast<uint2*>(r + 8u * (lane & 7u));
-    auto row = [&](uint32_t k, float v) {
+    auto row = [&](uint32_t i, float v) {
         const float v2 = v - top8(v);
-        rc[8u * k] = make_uint2(hi16_pair(v, v2), __float_as_uint(v2 - top8(v2)));
+        rc[8u * i] = make_uint2(hi16_pair(v, v2), __float_as_uint(v2 - top8(v2)));
     };
     row(0, c + p);
     row(1, c + q);
@@ -2070,23 +2073,23 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
     const PrimGeom* __restrict__ geom = in.geom;
     // The list is scanned 64 entries at a time with the entries' own bits
     // (the quadrant's bit, the depth key against qzmax); the entries that
-    // pass queue up in list order (in this wave's shading-colour row, which
-    // the shading stage fills only after the walk), and the record-based
-    // culls and the walk run on batches of queued candidates (the rest at
-    // the end of the list), so a long list with sparse candidates pays for
-    // them once per batch of candidates rather than once per 64 entries.
-    // A batch runs once QUEUE_RUN candidates are queued (up to 64 at once):
-    // waiting for fewer than 64 lets each walk tighten qzmax for the next
+    // pass queue up in list order (in LDS that the shading stage takes over
+    // after the walk), and the record-based culls and the walk run on batches
+    // of queued candidates (the rest at the end of the list), so a long list
+    // with sparse candidates pays for them once per batch of candidates rather
+    // than once per 64 entries.
+    // A batch runs once QUEUE_RUN candidates are queued (up to walk_batch at
+    // once): waiting for fewer lets each walk tighten qzmax for the next
     // entries sooner, which pays on short lists (batched scenes 1% faster at
     // 32 than at 64); long lists, with sparse candidates, do better with
     // fuller batches (the 1080p soup's raster 2.5% faster at 48 than at 32).
-    const uint32_t QUEUE_RUN = uniform(tr.z - tr.y) > 1024u ? 48u : 32u;
-    static_assert(48u + 63u <= WAVE_QUEUE, "candidate queue");
+    constexpr uint32_t BATCH = walk_batch(R);
+    const uint32_t QUEUE_RUN = R != 1 ? BATCH : (uniform(tr.z - tr.y) > 1024u ? BATCH : 32u);
     // the matrix path's right operand: X, X, X, Y, Y, Y, 0, 0 in the lanes of
     // the first eight k, 1, 1, 0, 1, 0... in the others
     MfmaIn cols;
     {
-        const float cx = (float)(8u * (lane & 7u)), cy = (float)(8u * ((lane >> 3) & 3u));
+        const float cx = (float)(int)(8u * (lane & 7u) - 28u), cy = (float)(int)(8u * ((lane >> 3) & 3u) - 12u);
         const uint4 v = lane < 32u ? make_uint4(hi16_pair(cx, cx), hi16_pair(cx, cy), hi16_pair(cy, cy), 0u)
                                    : make_uint4(hi16_pair(1.0f, 1.0f), hi16_pair(0.0f, 1.0f), 0u, 0u);
         __builtin_memcpy(&cols, &v, sizeof(cols));
@@ -2100,7 +2103,8 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
     WalkLds<R>& wl = sh.walk(row);
     constexpr uint32_t GROUP = walk_group(R);
     uint32_t* const cq = wl.queue;
-    uint32_t qn = 0;  // queued candidates (at most QUEUE_RUN + 63)
+    uint32_t qn = 0;  // queued candidates (at most BATCH + 63)
+    static_assert(sizeof(wl.queue) / 4u >= BATCH + 63u, "candidate queue");
     // this quadrant's bit in its fine tile's entries (its position in the
     // 32x32 fine tile, or in the 16x16 raster tile), and the key's bits
     const uint32_t qmask = 1u << (sc.fts == 5u ? ((((qy0 >> 3) & 3u) << 2) | ((qx0 >> 3) & 3u)) : wave);
@@ -2110,7 +2114,9 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
     // each 64 entries are loaded one step ahead
     uint32_t base = lbeg;
     for (;;) {
-        while (base < lend) {
+        // (a batch may leave QUEUE_RUN or more behind: it is followed by another
+        // before the list is read on, so qn stays within QUEUE_RUN + 63)
+        while (base < lend && qn < QUEUE_RUN) {
             const uint2 en = en_next;
             if (STATS) st_entries += min(64u, lend - base);
             base += 64;
@@ -2120,11 +2126,10 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
             const uint64_t mc = ballot(c0);
             if (c0) cq[qn + mbcnt(mc)] = en.x;
             qn += (uint32_t)__popcll(mc);
-            if (qn >= QUEUE_RUN) break;
         }
         if (qn == 0) break;
         // the next batch of queued candidates; the rest (< 64) move to the front
-        const uint32_t take = min(qn, 64u), left = qn - take;
+        const uint32_t take = min(qn, BATCH), left = qn - take;
         __builtin_amdgcn_wave_barrier();
         const uint32_t myprim = lane < take ? cq[lane] : 0u;
         if (left != 0) {
@@ -2143,8 +2148,8 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
             // depth lower bound over the quadrant's samples: the plane's smallest
             // value on the square through the outermost ones, and the vertices'
             const uint32_t bbx = __float_as_uint(g4.x), bby = __float_as_uint(g4.y);
-            const float zc = __builtin_fmaf(g3.y, qyc - g1.y, __builtin_fmaf(g3.x, qxc - g1.x, g3.w));
-            const float zq = __builtin_fmaf(-3.875f, fabsf(g3.x) + fabsf(g3.y), zc);
+            const float zr = __builtin_fmaf(g3.y, qyc - g1.y, g3.x * (qxc - g1.x));
+            const float zq = __builtin_fmaf(-3.875f, fabsf(g3.x) + fabsf(g3.y), zr + g3.w);
             // less what a stored depth may lie below its exact value
             lane_zlb = fmaxf(zq, g4.z) - 1.125f * WALK_EZ;
             {
@@ -2159,11 +2164,23 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
             // square through the quadrant's outermost samples (all lie within
             // 3.875 px of its centre), against the margin |rscale| scales to
             // WALK_TOL (a NaN where no margin is known: never culled)
-            const float e0 = corner_edge(g1.z, g1.w, g0.x, g0.y, qxc, qyc);
-            const float e1 = corner_edge(g2.x, g2.y, g0.z, g0.w, qxc, qyc);
-            const float e2 = corner_edge(g2.z, g2.w, g1.x, g1.y, qxc, qyc);
+            const float c0 = centre_edge(g1.z, g1.w, g0.x, g0.y, qxc, qyc);
+            const float c1 = centre_edge(g2.x, g2.y, g0.z, g0.w, qxc, qyc);
+            const float c2 = centre_edge(g2.z, g2.w, g1.x, g1.y, qxc, qyc);
+            const float e0 = __builtin_fmaf(3.875f, fabsf(g1.z) + fabsf(g1.w), c0);
+            const float e1 = __builtin_fmaf(3.875f, fabsf(g2.x) + fabsf(g2.y), c1);
+            const float e2 = __builtin_fmaf(3.875f, fabsf(g2.z) + fabsf(g2.w), c2);
             cand = (lane < take) & !(fminf(fminf(e0, e1), e2) * fabsf(g3.z) < -WALK_TOL) & !(lane_zlb >= qzmax);
             fast = g3.z > 0.0f;
+            // what walk_rows makes the prim's rows of: one load of the record
+            // serves both, and the walk waits for no memory
+            if (cand) {
+                const float s8 = g3.z * 0.125f;
+                WalkCoef& wc = wl.coef[lane];
+                wc.a = make_float4(g1.z * s8, g2.x * s8, g2.z * s8, g3.x * 0.125f);
+                wc.b = make_float4(g1.w * s8, g2.y * s8, g2.w * s8, g3.y * 0.125f);
+                wc.c = make_float4(c0 * g3.z, c1 * g3.z, c2 * g3.z, zr + g4.w);
+            }
         }
         uint64_t m = ballot(cand);
         const uint64_t mfast = ballot(fast);
@@ -2172,7 +2189,7 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
         while (m != 0) {
             // the next group: candidates in list order that some lane can still
             // take -- pixel inside the bbox and a stored depth above the bound
-            // (their lanes times 4, a byte each, in list order)
+            // (their lanes, a byte each, in list order)
             uint64_t group = 0, gfast = 0;
             uint32_t n8 = 0;  // 8 times their number
             do {
@@ -2180,7 +2197,7 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                 clear_bit(m, k);
                 const float zlb = __uint_as_float(lane_value(__float_as_uint(lane_zlb), k));
                 if ((ballot(!(zlb >= lane_zbmax)) & lane_value(lane_box, k)) != 0) {
-                    group |= (uint64_t)(4u * k) << n8;
+                    group |= (uint64_t)k << n8;
                     set_bit(gfast, k);
                     n8 += 8;
                     if (n8 == 8 * GROUP) break;
@@ -2191,16 +2208,14 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                 uint32_t l = lane;
                 asm volatile("" : "+v"(l));  // what follows from it is not held across the walk
                 const uint32_t src = (l >= 32u ? hi32(group) : lo32(group)) >> (l & 24u);
-                const uint32_t prim = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src & 0xFFu), (int)myprim);
-                if (GROUP == 8u || l < 8u * GROUP)
-                    walk_rows(geom, prim, wl.rows, l, (float)(8u * qx0 + 4u), (float)(8u * qy0 + 4u));
+                if (GROUP == 8u || l < 8u * GROUP) walk_rows(wl.coef, src & 0xFFu, wl.rows, l);
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             }
             const char* rp = reinterpret_cast<const char*>(wl.rows) + row_ofs;
             for (; n8 != 0; n8 -= 8, group >>= 8, rp += sizeof(WalkRows)) {
-                const uint32_t k = (lo32(group) & 0xFFu) >> 2;
+                const uint32_t k = lo32(group) & 0xFFu;
                 const uint32_t prim = lane_value(myprim, k);
                 bool exact = ((mfast >> k) & 1u) == 0;
                 if (!exact) {
@@ -2250,21 +2265,14 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                     }
                 }
                 if (exact) {
-                    // the reference's own steps, on exact stored depths
+                    // the reference's own steps
                     const uint64_t box = lane_value(lane_box, k);
                     const WalkRec gm = walk_rec(geom + prim);
                     uint32_t le = lane;
                     asm volatile("" : "+v"(le));  // the coordinates are not held across the walk
                     const float fx = (float)(qx0 + (le & 7)), fy = (float)(qy0 + (le >> 3));
                     float zs[4] = {zb0, zb1, zb2, zb3};
-                    if (approx) {
-                        const uint32_t wins[4] = {win0, win1, win2, win3};
-                        for (int q = 0; q < 4; ++q) {
-                            const uint32_t wp = PACKED ? packed_prim(wins[q]) : win[q * 64 + lane].x;
-                            if (wp != NO_PRIM) zs[q] = exact_depth(geom[wp], fx + sample_x(q), fy + sample_y(q));
-                        }
-                        approx = false;
-                    }
+                    const uint32_t wins[4] = {win0, win1, win2, win3};
                     // pixels inside the bbox (the others are not the prim's)
                     const bool live = (box >> lane) & 1u;
                     // mod.rs:134-146 + 148-170: coverage of the 4 samples
@@ -2288,6 +2296,12 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                         const float b1 = clamp_bary(e2 * gm.inv_area);
                         const float b2 = clamp_bary(1.0f - b0 - b1);
                         const float z = b0 * gm.z0 + b1 * gm.z1 + b2 * gm.z2;
+                        // a stored depth farther than its error from z decides as
+                        // its exact value would
+                        if (approx && ballot(in & (fabsf(z - zs[q]) <= 1.125f * WALK_EZ)) != 0) {
+                            const uint32_t wp = PACKED ? packed_prim(wins[q]) : win[q * 64 + lane].x;
+                            if (wp != NO_PRIM) zs[q] = exact_depth(geom[wp], sx, sy);
+                        }
                         if (in && z < zs[q]) {
                             zs[q] = z;
                             pass |= 1u << q;
@@ -2495,7 +2509,7 @@ __device__ __forceinline__ void report_job(const JobBufs& b) {
 // Persistent raster (raster_per_cu > 0): raster_per_cu workgroups of four
 // waves per CU, each wave one quadrant of the tile its workgroup holds;
 // contiguous bands of tiles become 8 queues, drained XCD-local first. Held
-// to 64 VGPRs (8 waves per SIMD), it keeps 40 bytes of its loop state per
+// to 64 VGPRs (8 waves per SIMD), it keeps 60 bytes of its loop state per
 // lane in scratch, and at 8 workgroups per CU runs a quarter faster than
 // unconstrained (6 waves).
 template <bool STATS>

@@ -62,16 +62,17 @@ def plane_of(p, n, inv, z, bbox):
     return F(lo), F(px), F(py), ez <= 0.9375 * EZ
 
 
-def rows(nx, ny, ax, ay, sc, c0, qx, qy):
-    """walk_rows(): coefficients A, B and the constant of each (half, sample)."""
-    s8 = F(sc * F(0.125))
+def rows(nx, ny, ax, ay, rs, z2, qx, qy):
+    """The candidate's coefficients about the quadrant's centre, then walk_rows():
+    A, B and the constant of each (half, sample). z2: None for an edge."""
+    s8 = F(rs * F(0.125))
     a, b = F(nx * s8), F(ny * s8)
-    dx, dy = fma(F(-8), ax, F(8 * qx + 4)), fma(F(-8), ay, F(8 * qy + 4))
-    c0 = fma(a, dx, fma(b, dy, c0))
+    c0 = fma(ny, F(F(qy + 4) - ay), F(nx * F(F(qx + 4) - ax)))
+    c0 = F(c0 * rs) if z2 is None else F(c0 + z2)
     p, q = fma(F(-3), b, a), fma(F(3), a, b)
     c = {}
     for h in (0, 1):
-        base = fma(F(32 * h), b, c0)
+        base = fma(F(32 * h - 16), b, c0)
         for k, v in ((0, F(base + p)), (1, F(base + q)), (2, F(base - p)), (3, F(base - q))):
             c[h, k] = v
     return float(a), float(b), c
@@ -111,14 +112,15 @@ def test_matrix_path_margins(kind):
         tie = [bool((nx > 0) or (not (nx < 0) and ny < 0)) for nx, ny in n]
         cx, cy, cz = covered_depths(p, n, inv, z, bbox, tie) if (bbox[1] - bbox[0]) * (bbox[3] - bbox[2]) < 10**5 else \
             [np.zeros(0, np.float32)] * 3
-        bound = fma(pzy, (cy - p[2][1]).astype(np.float32), fma(pzx, (cx - p[2][0]).astype(np.float32), pz0))
+        bound = fma(pzy, (cy - p[2][1]).astype(np.float32), (pzx * (cx - p[2][0]).astype(np.float32)).astype(np.float32))
+        bound = (bound + pz0).astype(np.float32)
         assert (cz >= bound).all(), kind
         below += cz.size
         rs = scale_of(p, n, bbox)
         fast += ok
         qs = [(x, y) for x in range(bbox[0] // 8 * 8, bbox[1], 8) for y in range(bbox[2] // 8 * 8, bbox[3], 8)]
         for qx, qy in [qs[i] for i in rng.permutation(len(qs))[:4]]:
-            fn = [rows(n[k][0], n[k][1], p[k][0], p[k][1], rs, F(0), qx, qy) for k in range(3)]
+            fn = [rows(n[k][0], n[k][1], p[k][0], p[k][1], rs, None, qx, qy) for k in range(3)]
             fn.append(rows(pzx, pzy, p[2][0], p[2][1], F(1), z[2], qx, qy))
             X, Y = np.meshgrid(np.arange(8), np.arange(8))
             for k in range(4):
@@ -128,7 +130,7 @@ def test_matrix_path_margins(kind):
                 for f in range(4):
                     a, b, c = fn[f]
                     cc = np.where(Y < 4, float(c[0, k]), float(c[1, k]))
-                    tx, ty = a * 8 * X, b * 8 * (Y % 4)
+                    tx, ty = a * (8 * X - 28), b * (8 * (Y % 4) - 12)
                     val.append(tx + ty + cc)
                     err.append(8 * U * (abs(tx) + abs(ty) + abs(cc)))
                 for f in range(3):
