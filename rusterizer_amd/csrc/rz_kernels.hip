@@ -2588,9 +2588,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
 // hold up all of them. Any grid of at least raster_grid_q(nt) workgroups
 // covers every quadrant; extra ones exit. Held to 64 VGPRs (8 waves per
 // SIMD): the extra waves hide more of the walk's load latency than anything
-// the limit costs.
+// the limit costs. The limit is given in registers (num_vgpr counts half of
+// the unified file): asked for as 8 waves, it would also hold the kernel to 80
+// SGPRs and move 28 of them through vector lanes; 94 leave it 8 waves and 2 such
+// moves (soup 0.353 -> 0.347 ms, 15,000 triangles 28.9 -> 28.0 us).
 template <bool STATS>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8, 8))) void k_raster_q(
+__global__ __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 7, 8), amdgpu_num_vgpr(32), amdgpu_num_sgpr(96))) void k_raster_q(
     JobBufs b, const PrimGeom* __restrict__ geom, const float* __restrict__ attrs, const float* __restrict__ uvat,
     const uint2* __restrict__ flist,
     const uint4* __restrict__ tile_rec, const SceneCfg* __restrict__ scenes, const DrawDev* __restrict__ draws) {
