@@ -964,8 +964,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         const SceneCfg& sc = scenes[scene];
         const SceneRun& run = runs[scene];
         const uint32_t W = sc.W, H = sc.H, fs = dd.fs;
-        // texel indices of this draw's texture fit 32-bit (24-bit factor) arithmetic
-        const bool tex_idx32 = dd.tw < (1u << 24) && dd.th < (1u << 24) && (uint64_t)dd.tw * dd.th <= 0xFFFFFFFFull;
+        // texel offsets of this draw's texture fit 32-bit (24-bit factor) arithmetic
+        const bool tex_idx32 = dd.tw < (1u << 24) && dd.th < (1u << 24) && (uint64_t)dd.tw * dd.th <= 1u << 30;
         const bool proofs = b.exact_paths == 0;
         // the chunk's prim range (its 256 triangles belong to draw d: draws are 256-aligned)
         const uint32_t blk_first = one ? s0 : uniform(run.prim_base + (s0 - run.prim_off));
@@ -1595,18 +1595,15 @@ __device__ __forceinline__ float sample_y(int s) {
     return s == 0 ? 0.125f : (s == 1 ? 0.625f : (s == 2 ? 0.875f : 0.375f));
 }
 
+typedef const __attribute__((address_space(1))) uint32_t* TexPtr;  // texels: global memory
+
 // texture.rs:47-63: linear texel index x + y*w; past the buffer -> last texel + flag
-__device__ __forceinline__ uint32_t read_texel(const uint32_t* __restrict__ tex, uint32_t tw, uint32_t th,
+__device__ __forceinline__ uint32_t read_texel(TexPtr tex, uint32_t tw, uint32_t th,
                                                uint32_t x, uint32_t y, bool& oob) {
-    uint64_t n = (uint64_t)tw * th;
-    uint64_t idx;
-    if (y >= th || (uint64_t)x >= n - (uint64_t)y * tw) {
-        oob = true;
-        idx = n - 1;
-    } else {
-        idx = (uint64_t)x + (uint64_t)y * tw;
-    }
-    return tex[idx];
+    const uint64_t n = (uint64_t)tw * th, row = (uint64_t)y * tw;
+    const bool past = (y >= th) | ((uint64_t)x >= n - row);
+    oob |= past;
+    return tex[past ? n - 1 : row + x];
 }
 
 struct RGBA {
@@ -1628,8 +1625,8 @@ __device__ constexpr ByteToFloat kByteToFloat = make_byte_to_float();
 
 // texture.rs:65-83 (channels via color.rs:22-29, byte / 255.0 from a table)
 // checked: bounds-checked texel reads (texture.rs:47-63); otherwise the prim's
-// coordinates are proven in bounds and the index x + y*tw fits 32 bits.
-__device__ __forceinline__ RGBA texture_sample(const uint32_t* __restrict__ tex, uint32_t tw, uint32_t th,
+// coordinates are proven in bounds and the byte offset 4 * (x + y*tw) fits 32 bits.
+__device__ __forceinline__ RGBA texture_sample(TexPtr tex, uint32_t tw, uint32_t th,
                                                float u, float v, const float* lut, bool checked, bool& oob) {
     float x = u * (float)(tw - 1);
     float y = v * (float)(th - 1);
@@ -1637,16 +1634,23 @@ __device__ __forceinline__ RGBA texture_sample(const uint32_t* __restrict__ tex,
     uint32_t yf0 = sat_u32(floorf(y)), yc = sat_u32(ceilf(y));
     uint32_t tl, tr, bl, br;
     if (checked) {
+        // (rare: one at a time, so that four 64-bit indices need no registers)
         tl = read_texel(tex, tw, th, xf0, yf0, oob);
+        asm volatile("" : "+v"(tl));
         tr = read_texel(tex, tw, th, xc, yf0, oob);
+        asm volatile("" : "+v"(tr));
         bl = read_texel(tex, tw, th, xf0, yc, oob);
+        asm volatile("" : "+v"(bl));
         br = read_texel(tex, tw, th, xc, yc, oob);
     } else {
         const uint32_t r0 = __umul24(yf0, tw), r1 = __umul24(yc, tw);
-        tl = tex[r0 + xf0];
-        tr = tex[r0 + xc];
-        bl = tex[r1 + xf0];
-        br = tex[r1 + xc];
+        const auto texel = [&](uint32_t i) {  // the byte offset fits 32 bits, added to a uniform base
+            return *(TexPtr)((const __attribute__((address_space(1))) char*)tex + 4u * i);
+        };
+        tl = texel(r0 + xf0);
+        tr = texel(r0 + xc);
+        bl = texel(r1 + xf0);
+        br = texel(r1 + xc);
     }
     float x_f = x - truncf(x);
     float y_f = y - truncf(y);
@@ -1689,9 +1693,10 @@ __device__ __forceinline__ float centre_edge(float nx, float ny, float ax, float
     return __builtin_fmaf(ny, yc - ay, nx * (xc - ax));
 }
 
-// bits 0..3 of v as bytes 0x00 or 0xFF
-__device__ __forceinline__ uint32_t bits_to_bytes(uint32_t v) {
-    return (__umul24(v, 0x204081u) & 0x01010101u) * 0xFFu;
+// byte 0 of row in the bytes whose bit in skip (4 bits) is clear, 0 in the others
+__device__ __forceinline__ uint32_t spread_row(uint32_t row, uint32_t skip) {
+    // a byte select of 4 takes a byte of the first argument
+    return __builtin_amdgcn_perm(0u, row, __umul24(skip, 0x810204u) & 0x04040404u);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -1745,12 +1750,11 @@ __device__ __forceinline__ uint32_t band_lo(uint32_t nt, uint32_t x) {
 // first passing sample
 __device__ __forceinline__ void frag_bary(const PrimGeom& g, float fx, float fy, uint32_t pass, float& u, float& v,
                                           float& w) {
-    float ix = fx + 0.5f, iy = fy + 0.5f;
-    if (pass != 0xFu) {
-        const int k = __builtin_ctz(pass);
-        ix = fx + sample_x(k);
-        iy = fy + sample_y(k);
-    }
+    // nibble k: sample k's offset in eighths of a pixel, nibble 4 the centre's
+    // (the products are exact)
+    const uint32_t k4 = pass == 0xFu ? 16u : 4u * (uint32_t)__builtin_ctz(pass);
+    const float ix = __builtin_fmaf((float)(0x41375u >> k4 & 7u), 0.125f, fx);
+    const float iy = __builtin_fmaf((float)(0x43751u >> k4 & 7u), 0.125f, fy);
     const float ef0 = edge(g.nx0, g.ny0, g.ax0, g.ay0, ix, iy);
     const float ef1 = edge(g.nx1, g.ny1, g.ax1, g.ay1, ix, iy);
     const float ef2 = edge(g.nx2, g.ny2, g.ax2, g.ay2, ix, iy);
@@ -1794,15 +1798,17 @@ __device__ __forceinline__ float sample0_depth(const PrimGeom& g, float fx, floa
 
 // the texture of a scene with a single, textured draw (tex null: look at each
 // prim's draw): known before the prims' records, in scalar registers
+typedef const __attribute__((address_space(4))) SceneCfg* SceneTable;
+typedef const __attribute__((address_space(4))) DrawDev* DrawTable;
 struct DrawTex {
-    const uint32_t* tex;
+    TexPtr tex;
     uint32_t tw, th;
 };
 
 // main.rs:67-77 fragment shaders, then mod.rs:380-397 (to ARGB): the colour
 // one fragment writes to its passing samples
 __device__ __forceinline__ uint32_t shade_fragment(const PrimGeom& g, const float* __restrict__ at,
-                                                   const float* __restrict__ uv, const DrawDev* __restrict__ draws,
+                                                   const float* __restrict__ uv, DrawTable draws,
                                                    const DrawTex& only, float fx, float fy, uint32_t pass, const float* lut, bool& oob) {
     float u, v, w;
     frag_bary(g, fx, fy, pass, u, v, w);
@@ -1821,8 +1827,8 @@ __device__ __forceinline__ uint32_t shade_fragment(const PrimGeom& g, const floa
         if (only.tex) {
             c = texture_sample(only.tex, only.tw, only.th, tu, tv, lut, checked, oob);
         } else {
-            const DrawDev& dd = draws[g.flags >> 16];
-            c = texture_sample(dd.tex, dd.tw, dd.th, tu, tv, lut, checked, oob);
+            const auto& dd = draws[g.flags >> 16];
+            c = texture_sample((TexPtr)dd.tex, dd.tw, dd.th, tu, tv, lut, checked, oob);
         }
         cr = c.r; cg = c.g; cbl = c.b; ca = c.a;
     } else {  // Debug: Color::grayscale(depths[0]) (color.rs:65-72)
@@ -1837,12 +1843,20 @@ __device__ __forceinline__ uint32_t shade_fragment(const PrimGeom& g, const floa
 // records with scalar loads while the kernel writes its outputs.
 struct RasterIn {
     const PrimGeom* __restrict__ geom;
-    const float* __restrict__ attrs;
-    const float* __restrict__ uvat;
     const uint2* __restrict__ flist;
     const uint4* __restrict__ tile_rec;
     const SceneCfg* __restrict__ scenes;
-    const DrawDev* __restrict__ draws;
+};
+// What is used after the walk (and by rare prims in it). No kernel writes the
+// tables while a raster runs, so they are read through the constant address
+// space, with scalar loads where the record is uniform.
+struct RasterLate {
+    const float* attrs;
+    const float* uvat;
+    DrawTable draws;
+    SceneTable scenes;
+    SceneRun* runs;
+    uint32_t* host_oob;
 };
 
 // The words of a prim record that the exact path reads, as scalars.
@@ -1878,10 +1892,10 @@ static_assert(offsetof(PrimGeom, nx0) == 24 && offsetof(PrimGeom, pzx) == 48 && 
 // The walk is bound by instruction issue: a prim takes 35 vector instructions
 // here against about 120 by the reference's steps; 2 to 13% of the prims take
 // those, and look up an exact stored depth only for samples where it decides.
-// Raster of 256 textured scenes 6.55 -> 5.00 ms (5.21 with every stored depth
+// Raster of 256 textured scenes 6.55 -> 4.79 ms (5.21 against 5.00 with every stored depth
 // made exact for each such prim and the records loaded again for the rows), of
-// a 1M-triangle 1080p soup 0.419 -> 0.341 ms, of a 4M-triangle 4K terrain
-// 0.348 -> 0.220 ms. Groups of 8 prims against 4: the
+// a 1M-triangle 1080p soup 0.419 -> 0.331 ms, of a 4M-triangle 4K terrain
+// 0.348 -> 0.210 ms. Groups of 8 prims against 4: the
 // terrain's 0.217 against 0.234 ms, the batch the same.
 typedef float MfmaAcc __attribute__((ext_vector_type(16)));
 typedef __bf16 MfmaIn __attribute__((ext_vector_type(8)));
@@ -2019,9 +2033,10 @@ __device__ __forceinline__ float exact_depth(const PrimGeom& g, float sx, float 
 // R = 4: the workgroup's four waves take the tile's four quadrants and
 // share the shading tasks; R = 1: the workgroup is one wave and takes
 // quadrant quad of the tile alone.
-template <bool STATS, uint32_t R>
-__device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, const RasterIn& in, uint32_t slot, uint32_t quad, uint4 tr1,
-                                            float* lut, ShadeLds<R>& sh,
+// late(): the RasterLate, fetched where it is used.
+template <bool STATS, uint32_t R, class Late>
+__device__ __forceinline__ void raster_tile(const Late& late, const RasterIn& in, uint32_t slot, uint32_t quad,
+                                            uint4 tr1, float* lut, ShadeLds<R>& sh,
                                             uint32_t& st_entries, uint32_t& st_cand, uint32_t& st_hits,
                                             uint32_t& st_cov, uint32_t& st_shaded) {
     // the tile's scene and this wave's list range (k_tile_prep)
@@ -2099,7 +2114,8 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
     // zero beside what follows either
     const uint32_t row_ofs = lane < 32u ? (uint32_t)offsetof(WalkRows, ab) + 16u * (lane & 3u) : 8u * (lane & 31u);
     const float inf = opaque_inf();
-    bool approx = false;  // some stored depth may be off by up to WALK_EZ
+    // (flags of the whole wave: kept as numbers, which take one scalar register)
+    uint32_t approx = 0;  // some stored depth may be off by up to WALK_EZ
     WalkLds<R>& wl = sh.walk(row);
     constexpr uint32_t GROUP = walk_group(R);
     uint32_t* const cq = wl.queue;
@@ -2155,10 +2171,9 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
             {
                 const uint32_t cx0 = min(max(bbx & 0xFFFFu, qx0) - qx0, 8u), cx1 = min(max(bbx >> 16, qx0) - qx0, 8u);
                 const uint32_t cy0 = min(max(bby & 0xFFFFu, qy0) - qy0, 8u), cy1 = min(max(bby >> 16, qy0) - qy0, 8u);
-                // one row's columns in every byte, kept in the bytes of rows cy0..cy1 - 1
-                const uint32_t row = __builtin_amdgcn_perm(0u, (1u << cx1) - (1u << cx0), 0u);
-                const uint32_t rows = (1u << cy1) - (1u << cy0);
-                lane_box = (uint64_t)(row & bits_to_bytes(rows >> 4)) << 32 | (row & bits_to_bytes(rows & 15u));
+                // one row's columns in the bytes of rows cy0..cy1 - 1
+                const uint32_t row = (1u << cx1) - (1u << cx0), skip = ~((1u << cy1) - (1u << cy0));
+                lane_box = (uint64_t)spread_row(row, skip >> 4 & 15u) << 32 | spread_row(row, skip & 15u);
             }
             // the largest value of the edges that is the smallest, over the
             // square through the quadrant's outermost samples (all lie within
@@ -2185,7 +2200,7 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
         uint64_t m = ballot(cand);
         const uint64_t mfast = ballot(fast);
         if (STATS) st_cand += (uint32_t)__popcll(m);
-        bool dirty = false;
+        uint32_t dirty = 0;
         while (m != 0) {
             // the next group: candidates in list order that some lane can still
             // take -- pixel inside the bbox and a stored depth above the bound
@@ -2260,7 +2275,7 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                             zb1 = p1 ? d[7] : zb1;
                             zb2 = p2 ? d[11] : zb2;
                             zb3 = p3 ? d[15] : zb3;
-                            dirty = approx = true;
+                            dirty = approx = 1u;
                         }
                     }
                 }
@@ -2298,7 +2313,7 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                         const float z = b0 * gm.z0 + b1 * gm.z1 + b2 * gm.z2;
                         // a stored depth farther than its error from z decides as
                         // its exact value would
-                        if (approx && ballot(in & (fabsf(z - zs[q]) <= 1.125f * WALK_EZ)) != 0) {
+                        if (approx != 0 && ballot(in & (fabsf(z - zs[q]) <= 1.125f * WALK_EZ)) != 0) {
                             const uint32_t wp = PACKED ? packed_prim(wins[q]) : win[q * 64 + lane].x;
                             if (wp != NO_PRIM) zs[q] = exact_depth(geom[wp], sx, sy);
                         }
@@ -2318,8 +2333,9 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                             // fragment, also ones overwritten later)
                             float u, v, w;
                             frag_bary(geom[prim], fx, fy, pass, u, v, w);
-                            const float* at = in.uvat + (size_t)prim * UV_STRIDE;
-                            const DrawDev& dd = in.draws[gm.flags >> 16];
+                            const RasterLate la = late();
+                            const float* at = la.uvat + (size_t)prim * UV_STRIDE;
+                            const auto& dd = la.draws[gm.flags >> 16];
                             oob |= texel_oob(dd.tw, dd.th, at[0] * u + at[2] * v + at[4] * w,
                                              at[1] * u + at[3] * v + at[5] * w);
                         }
@@ -2342,15 +2358,20 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                     zb1 = zs[1];
                     zb2 = zs[2];
                     zb3 = zs[3];
-                    dirty = true;
+                    dirty = 1u;
                 }
             }
             lane_zbmax = max_raw(max_raw(zb0, zb1, inf), max_raw(zb2, zb3, inf), inf);
         }
         // stored depths only fall, so a stale qzmax is still an upper bound;
         // it is refreshed once per batch of entries
-        if (dirty) qzmax = wave_max_uniform(lane_zbmax, inf) + 1.125f * WALK_EZ;
+        if (dirty != 0) qzmax = wave_max_uniform(lane_zbmax, inf) + 1.125f * WALK_EZ;
     }
+    const RasterLate la = late();
+    uint32_t sid = s;
+    asm volatile("" : "+s"(sid));  // addresses are formed here, not held across the walk
+    const auto& so = la.scenes[sid];
+    const uint32_t W2 = so.W, H2 = so.H;
     {
         // the pixel's coordinates are recomputed here and below rather than
         // held across the walk and the shading (registers are the raster's
@@ -2358,8 +2379,8 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
         uint32_t l2 = lane;
         asm volatile("" : "+v"(l2));
         const uint32_t px2 = qx0 + (l2 & 7), py2 = qy0 + (l2 >> 3);
-        if (px2 < W && py2 < H && sc.msaa_depth) {
-            if (approx) {
+        if (px2 < W2 && py2 < H2 && so.msaa_depth) {
+            if (approx != 0) {
                 const float fx2 = (float)px2, fy2 = (float)py2;
                 float* const zs[4] = {&zb0, &zb1, &zb2, &zb3};
                 const uint32_t wins[4] = {win0, win1, win2, win3};
@@ -2370,13 +2391,13 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                 }
             }
             const float4 d4 = make_float4(zb0, zb1, zb2, zb3);
-            *reinterpret_cast<float4*>(sc.msaa_depth + ((size_t)py2 * W + px2) * 4) = d4;
+            *reinterpret_cast<float4*>(so.msaa_depth + ((size_t)py2 * W2 + px2) * 4) = d4;
         }
     }
     DrawTex only{nullptr, 0, 0};
-    if (sc.draw != MANY_DRAWS) {
-        const DrawDev& dd = in.draws[sc.draw];
-        only = DrawTex{dd.tex, dd.tw, dd.th};
+    if (so.draw != MANY_DRAWS) {
+        const auto& dd = la.draws[so.draw];
+        only = DrawTex{(TexPtr)dd.tex, dd.tw, dd.th};
     }
     // deferred shading: one task per distinct surviving prim of a pixel (its
     // first sample heads it); the workgroup's tasks are shaded 64 at a time
@@ -2436,8 +2457,18 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
             const uint32_t P = t.x, ol = t.y & 63u, pass = t.y >> 6;
             const float ofx = (float)(qx0 + (ol & 7u)), ofy = (float)(qy0 + (ol >> 3));
             const PrimGeom gp = geom[P];
-            sh.argb(0)[g] = shade_fragment(gp, in.attrs + (size_t)P * ATTR_STRIDE, in.uvat + (size_t)P * UV_STRIDE,
-                                           in.draws, only, ofx, ofy, pass, lut, oob);
+            if (only.tex) {
+                // a single textured draw: its coordinates are asked for beside the record
+                const float2* const ua = reinterpret_cast<const float2*>(la.uvat + (size_t)P * UV_STRIDE);
+                const float2 t0 = ua[0], t1 = ua[1], t2 = ua[2];
+                float u, v, w;
+                frag_bary(gp, ofx, ofy, pass, u, v, w);
+                const RGBA c = texture_sample(only.tex, only.tw, only.th, t0.x * u + t1.x * v + t2.x * w,
+                                              t0.y * u + t1.y * v + t2.y * w, lut, (gp.flags & PRIM_UV_CHECK) != 0, oob);
+                sh.argb(0)[g] = to_argb(c.r, c.g, c.b, c.a);
+            } else
+            sh.argb(0)[g] = shade_fragment(gp, la.attrs + (size_t)P * ATTR_STRIDE, la.uvat + (size_t)P * UV_STRIDE,
+                                           la.draws, only, ofx, ofy, pass, lut, oob);
             if (STATS) st_shaded += 1;  // shading tasks run by this lane
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -2460,7 +2491,7 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
                 const float ofy = (float)(ty * 16 + (r >> 1) * 8 + (ol >> 3));
                 const PrimGeom gp = geom[P];
                 sh.argb(r)[i] =
-                    shade_fragment(gp, in.attrs + (size_t)P * ATTR_STRIDE, in.uvat + (size_t)P * UV_STRIDE, in.draws,
+                    shade_fragment(gp, la.attrs + (size_t)P * ATTR_STRIDE, la.uvat + (size_t)P * UV_STRIDE, la.draws,
                                    only, ofx, ofy, pass, lut, oob);
                 if (STATS) st_shaded += 1;  // shading tasks run by this lane
             }
@@ -2473,22 +2504,22 @@ __device__ __forceinline__ void raster_tile(SceneRun* runs, uint32_t* host_oob, 
     const uint32_t cb2 = (vmask & 4u) ? wargb[(slots >> 16) & 0xFFu] : CLEAR_COLOR;
     const uint32_t cb3 = (vmask & 8u) ? wargb[slots >> 24] : CLEAR_COLOR;
     if (ballot(oob) && lane == 0) {
-        atomicOr(&runs[s].flags, RZ_FLAG_TEXEL_OOB);
-        if (host_oob) host_oob[s] = 1u;
+        atomicOr(&la.runs[sid].flags, RZ_FLAG_TEXEL_OOB);
+        if (la.host_oob) la.host_oob[sid] = 1u;
     }
     uint32_t l3 = lane;
     asm volatile("" : "+v"(l3));
     const uint32_t px3 = qx0 + (l3 & 7), py3 = qy0 + (l3 >> 3);
-    if (px3 < W && py3 < H) {
+    if (px3 < W2 && py3 < H2) {
         // buffers.rs:111-125: each channel's sum / 4, red and blue in 16-bit fields
         constexpr uint32_t RB = 0x00FF00FFu;
         const uint32_t rb = (cb0 & RB) + (cb1 & RB) + (cb2 & RB) + (cb3 & RB);
         const uint32_t gs = ((cb0 >> 8) & 0xFFu) + ((cb1 >> 8) & 0xFFu) + ((cb2 >> 8) & 0xFFu) + ((cb3 >> 8) & 0xFFu);
-        size_t o = (size_t)py3 * W + px3;
-        sc.out[o] = (0xFFu << 24) | ((rb >> 2) & RB) | (gs >> 2) << 8;
-        if (sc.msaa_color) {
+        size_t o = (size_t)py3 * W2 + px3;
+        so.out[o] = (0xFFu << 24) | ((rb >> 2) & RB) | (gs >> 2) << 8;
+        if (so.msaa_color) {
             uint4 c4 = make_uint4(cb0, cb1, cb2, cb3);
-            *reinterpret_cast<uint4*>(sc.msaa_color + o * 4) = c4;
+            *reinterpret_cast<uint4*>(so.msaa_color + o * 4) = c4;
         }
     }
 }
@@ -2517,7 +2548,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
     JobBufs b, const PrimGeom* __restrict__ geom, const float* __restrict__ attrs, const float* __restrict__ uvat,
     const uint2* __restrict__ flist,
     const uint4* __restrict__ tile_rec, const SceneCfg* __restrict__ scenes, const DrawDev* __restrict__ draws) {
-    const RasterIn in{geom, attrs, uvat, flist, tile_rec, scenes, draws};
+    const RasterIn in{geom, flist, tile_rec, scenes};
+    const auto late = [&] { return RasterLate{attrs, uvat, (DrawTable)draws, (SceneTable)scenes, b.runs, b.host_oob}; };
     __shared__ float lut[256];
     __shared__ uint32_t next_tile;
     __shared__ ShadeLds<4> sh;
@@ -2544,7 +2576,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
         const uint32_t tile = next_tile;
         __syncthreads();
         if (tile == NO_TILE) break;
-        raster_tile<STATS, 4>(b.runs, b.host_oob, in, tile, 0u, uint4{}, lut, sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
+        raster_tile<STATS, 4>(late, in, tile, 0u, uint4{}, lut, sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
     }
     if (STATS) {  // the last two counts are per lane
         for (int o = 32; o >= 1; o >>= 1) {
@@ -2588,17 +2620,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
 // hold up all of them. Any grid of at least raster_grid_q(nt) workgroups
 // covers every quadrant; extra ones exit. Held to 64 VGPRs (8 waves per
 // SIMD): the extra waves hide more of the walk's load latency than anything
-// the limit costs. The limit is given in registers (num_vgpr counts half of
-// the unified file): asked for as 8 waves, it would also hold the kernel to 80
-// SGPRs and move 28 of them through vector lanes; 94 leave it 8 waves and 2 such
-// moves (soup 0.353 -> 0.347 ms, 15,000 triangles 28.9 -> 28.0 us).
+// the limit costs. Eight waves also leave it 80 scalar registers: what does
+// not fit moves through vector lanes, which the vector units pay for (28 moved
+// registers took 5% of their instructions; seven waves with 94 scalar
+// registers: 5.00 against 4.82 ms for 256 textured scenes).
+//
+// Its arguments as they lie in memory: what only the shading needs is read
+// there after the walk, so that no scalar registers hold it meanwhile.
+struct RasterArgs {
+    JobBufs b;
+    const PrimGeom* geom;
+    const float* attrs;
+    const float* uvat;
+    const uint2* flist;
+    const uint4* tile_rec;
+    const SceneCfg* scenes;
+    const DrawDev* draws;
+};
 template <bool STATS>
-__global__ __launch_bounds__(64)
-    __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 7, 8), amdgpu_num_vgpr(32), amdgpu_num_sgpr(96))) void k_raster_q(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8, 8))) void k_raster_q(
     JobBufs b, const PrimGeom* __restrict__ geom, const float* __restrict__ attrs, const float* __restrict__ uvat,
     const uint2* __restrict__ flist,
     const uint4* __restrict__ tile_rec, const SceneCfg* __restrict__ scenes, const DrawDev* __restrict__ draws) {
-    const RasterIn in{geom, attrs, uvat, flist, tile_rec, scenes, draws};
+    const RasterIn in{geom, flist, tile_rec, scenes};
+    const auto late = [] {
+        typedef const __attribute__((address_space(4))) RasterArgs* Args;
+        Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));  // loaded here, not at the kernel's start
+        return RasterLate{a->attrs, a->uvat, (DrawTable)a->draws, (SceneTable)a->scenes, a->b.runs, a->b.host_oob};
+    };
     __shared__ ShadeLds<1> sh;
     constexpr uint32_t QRUN = 4u * RASTER_RUN;
     const uint32_t k = blockIdx.x >> 3, xcd = blockIdx.x & 7u;
@@ -2610,7 +2660,7 @@ __global__ __launch_bounds__(64)
     if (uniform(b.cnt->overflow) != 0) return;
     uint32_t st_entries = 0, st_cand = 0, st_hits = 0, st_cov = 0, st_shaded = 0;
     if (qs < nq)
-        raster_tile<STATS, 1>(b.runs, b.host_oob, in, qs >> 2, qs & 3u, tr, sh.lut(), sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
+        raster_tile<STATS, 1>(late, in, qs >> 2, qs & 3u, tr, sh.lut(), sh, st_entries, st_cand, st_hits, st_cov, st_shaded);
     if (STATS) {  // every workgroup writes its counts, zeros past the last quadrant
         for (int o = 32; o >= 1; o >>= 1) {  // the last two counts are per lane
             st_cov += __shfl_xor(st_cov, o);
@@ -2930,11 +2980,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             continue;
         }
         SvcJob* j = &ents[e].job;
-        const RasterIn in{svc_ptr<PrimGeom>(&j->geom), svc_ptr<float>(&j->attrs), svc_ptr<float>(&j->uvat),
-                          svc_ptr<uint2>(&j->flist),   svc_ptr<uint4>(&j->tile_rec), svc_ptr<SceneCfg>(&j->scenes),
-                          svc_ptr<DrawDev>(&j->draws)};
-        SceneRun* runs = svc_ptr_mut<SceneRun>(&j->runs);
-        raster_tile<false, 4>(runs, nullptr, in, t, 0u, uint4{}, lut, sh, st0, st1, st2, st3, st4);
+        const RasterIn in{svc_ptr<PrimGeom>(&j->geom), svc_ptr<uint2>(&j->flist), svc_ptr<uint4>(&j->tile_rec),
+                          svc_ptr<SceneCfg>(&j->scenes)};
+        const RasterLate rest{svc_ptr<float>(&j->attrs),
+                              svc_ptr<float>(&j->uvat),
+                              (DrawTable)svc_ptr<DrawDev>(&j->draws),
+                              (SceneTable)in.scenes,
+                              svc_ptr_mut<SceneRun>(&j->runs),
+                              nullptr};
+        const auto late = [&] { return rest; };
+        raster_tile<false, 4>(late, in, t, 0u, uint4{}, lut, sh, st0, st1, st2, st3, st4);
         pend_e = e;
         pend_g = g;
         pend_nt = nt;
