@@ -532,7 +532,9 @@ int size_buffers(rz_ctx* c, const JobPlan& pl, const Needs& n_in, G& g) {
     const size_t cls = g(c->cls, std::max<uint64_t>(NT, 256));
     g(c->nsub, cls);
     g(c->wave_prims, cls / 64 + 4);
-    if (pl.direct) g(c->wave_pairs, cls / 64 + 4);
+    // (only direct jobs use it; grown with the others, so that a small job after
+    // a large one never waits for a running raster service to free memory)
+    g(c->wave_pairs, cls / 64 + 4);
     g(c->chunk_off, cls / TRI_ALIGN + 1);
     const size_t geom = g(c->geom, n.prims);
     g(c->attrs, geom * ATTR_STRIDE);

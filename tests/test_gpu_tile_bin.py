@@ -86,3 +86,20 @@ def test_tile_bin_frames_of_many_draws(draws):
         parts = [_frame(1, 90, 50, 25, seed=1)]
         parts[0].idx = parts[0].idx[:0]
     assert_parity(run_gpu(parts), run_oracle(parts), where=f"{draws} draws")
+
+
+@pytest.mark.parametrize("small", [1, 300, 16384])
+def test_small_job_after_a_large_one_allocates_nothing(small):
+    """A context that has run a large job runs a small one in the buffers it
+    has: growing one waits for all work on the device (for a running raster
+    service to go idle, a tenth of a second)."""
+    from rusterizer_amd.render import Context
+
+    ctx = Context(64, 64)
+    try:
+        run_batch([_frame(140000, 320, 240, 1, seed=3)], ctx=ctx)
+        held = ctx.memory()["held"]
+        run_batch([_frame(small, 320, 240, 4, seed=4)], ctx=ctx)
+        assert ctx.memory()["held"] == held
+    finally:
+        ctx.close()
