@@ -12,7 +12,8 @@
 //   -> k_fine_prep -> scan64 -> k_fine_bin<count> -> scan
 //   -> k_fine_bin<scatter>                      (8, 16 or 32 px fine tiles)
 //   -> k_tile_prep -> k_raster_q (coverage, depth, shading, resolve)
-// (small jobs: k_tile_bin in place of both binning levels and k_tile_prep)
+// (small scenes: k_tile_bin in place of both binning levels and k_tile_prep;
+// one small scene: k_setup does k_scene_prep's work)
 // Rasterizer triangles ("prims") are stored per scene in submission order
 // (draw, input triangle, clip-fan index), so every later stage keeps the
 // reference's order per pixel without sorting. Each scene's prims start at a
@@ -1914,11 +1915,11 @@ static_assert(offsetof(PrimGeom, nx0) == 24 && offsetof(PrimGeom, pzx) == 48 && 
 // The walk is bound by instruction issue: a prim takes 35 vector instructions
 // here against about 120 by the reference's steps; 2 to 13% of the prims take
 // those, and look up an exact stored depth only for samples where it decides.
-// Raster of 256 textured scenes 6.55 -> 4.79 ms (5.21 against 5.00 with every stored depth
-// made exact for each such prim and the records loaded again for the rows), of
-// a 1M-triangle 1080p soup 0.419 -> 0.331 ms, of a 4M-triangle 4K terrain
-// 0.348 -> 0.210 ms. Groups of 8 prims against 4: the
-// terrain's 0.217 against 0.234 ms, the batch the same.
+// Raster of 256 textured scenes 6.55 -> 4.79 ms, of a 1M-triangle 1080p soup
+// 0.419 -> 0.331 ms, of a 4M-triangle 4K terrain 0.348 -> 0.210 ms. (Every
+// stored depth made exact for each such prim, and the records loaded again for
+// the rows: the batch's 5.21 ms where this form took 5.00.) Groups of 8 prims
+// against 4: the terrain's 0.217 against 0.234 ms, the batch the same.
 typedef float MfmaAcc __attribute__((ext_vector_type(16)));
 typedef __bf16 MfmaIn __attribute__((ext_vector_type(8)));
 // prims whose rows are prepared together: 8 lanes each, so 8 fill a wave; four-wave
@@ -2562,9 +2563,8 @@ __device__ __forceinline__ void report_job(const JobBufs& b) {
 // Persistent raster (raster_per_cu > 0): raster_per_cu workgroups of four
 // waves per CU, each wave one quadrant of the tile its workgroup holds;
 // contiguous bands of tiles become 8 queues, drained XCD-local first. Held
-// to 64 VGPRs (8 waves per SIMD), it keeps 60 bytes of its loop state per
-// lane in scratch, and at 8 workgroups per CU runs a quarter faster than
-// unconstrained (6 waves).
+// to 64 VGPRs (8 waves per SIMD), at 8 workgroups per CU it runs a quarter
+// faster than unconstrained (6 waves).
 template <bool STATS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8, 8))) void k_raster(
     JobBufs b, const PrimGeom* __restrict__ geom, const float* __restrict__ attrs, const float* __restrict__ uvat,
