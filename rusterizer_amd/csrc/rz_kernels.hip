@@ -1830,8 +1830,9 @@ struct DrawTex {
 
 // main.rs:67-77 fragment shaders, then mod.rs:380-397 (to ARGB): the colour
 // one fragment writes to its passing samples
+template <class Draws>
 __device__ __forceinline__ uint32_t shade_fragment(const PrimGeom& g, const float* __restrict__ at,
-                                                   const float* __restrict__ uv, DrawTable draws,
+                                                   const float* __restrict__ uv, Draws draws,
                                                    const DrawTex& only, float fx, float fy, uint32_t pass, const float* lut, bool& oob) {
     float u, v, w;
     frag_bary(g, fx, fy, pass, u, v, w);
@@ -1871,16 +1872,19 @@ struct RasterIn {
     const SceneCfg* __restrict__ scenes;
 };
 // What is used after the walk (and by rare prims in it). No kernel writes the
-// tables while a raster runs, so they are read through the constant address
-// space, with scalar loads where the record is uniform.
+// tables while a raster launched for one job runs, so it reads them through the
+// constant address space, with scalar loads where the record is uniform. The
+// raster service, whose tables change while it runs, takes plain pointers.
+template <class Scenes, class Draws>
 struct RasterLate {
     const float* attrs;
     const float* uvat;
-    DrawTable draws;
-    SceneTable scenes;
+    Draws draws;
+    Scenes scenes;
     SceneRun* runs;
     uint32_t* host_oob;
 };
+typedef RasterLate<SceneTable, DrawTable> JobLate;
 
 // The words of a prim record that the exact path reads, as scalars.
 struct WalkRec {
@@ -2356,7 +2360,7 @@ __device__ __forceinline__ void raster_tile(const Late& late, const RasterIn& in
                             // fragment, also ones overwritten later)
                             float u, v, w;
                             frag_bary(geom[prim], fx, fy, pass, u, v, w);
-                            const RasterLate la = late();
+                            const auto la = late();
                             const float* at = la.uvat + (size_t)prim * UV_STRIDE;
                             const auto& dd = la.draws[gm.flags >> 16];
                             oob |= texel_oob(dd.tw, dd.th, at[0] * u + at[2] * v + at[4] * w,
@@ -2390,7 +2394,7 @@ __device__ __forceinline__ void raster_tile(const Late& late, const RasterIn& in
         // it is refreshed once per batch of entries
         if (dirty != 0) qzmax = wave_max_uniform(lane_zbmax, inf) + 1.125f * WALK_EZ;
     }
-    const RasterLate la = late();
+    const auto la = late();
     uint32_t sid = s;
     asm volatile("" : "+s"(sid));  // addresses are formed here, not held across the walk
     const auto& so = la.scenes[sid];
@@ -2571,7 +2575,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
     const uint2* __restrict__ flist,
     const uint4* __restrict__ tile_rec, const SceneCfg* __restrict__ scenes, const DrawDev* __restrict__ draws) {
     const RasterIn in{geom, flist, tile_rec, scenes};
-    const auto late = [&] { return RasterLate{attrs, uvat, (DrawTable)draws, (SceneTable)scenes, b.runs, b.host_oob}; };
+    const auto late = [&] { return JobLate{attrs, uvat, (DrawTable)draws, (SceneTable)scenes, b.runs, b.host_oob}; };
     __shared__ float lut[256];
     __shared__ uint32_t next_tile;
     __shared__ ShadeLds<4> sh;
@@ -2669,7 +2673,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 
         typedef const __attribute__((address_space(4))) RasterArgs* Args;
         Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(a));  // loaded here, not at the kernel's start
-        return RasterLate{a->attrs, a->uvat, (DrawTable)a->draws, (SceneTable)a->scenes, a->b.runs, a->b.host_oob};
+        return JobLate{a->attrs, a->uvat, (DrawTable)a->draws, (SceneTable)a->scenes, a->b.runs, a->b.host_oob};
     };
     __shared__ ShadeLds<1> sh;
     constexpr uint32_t QRUN = 4u * RASTER_RUN;
@@ -3004,12 +3008,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         SvcJob* j = &ents[e].job;
         const RasterIn in{svc_ptr<PrimGeom>(&j->geom), svc_ptr<uint2>(&j->flist), svc_ptr<uint4>(&j->tile_rec),
                           svc_ptr<SceneCfg>(&j->scenes)};
-        const RasterLate rest{svc_ptr<float>(&j->attrs),
-                              svc_ptr<float>(&j->uvat),
-                              (DrawTable)svc_ptr<DrawDev>(&j->draws),
-                              (SceneTable)in.scenes,
-                              svc_ptr_mut<SceneRun>(&j->runs),
-                              nullptr};
+        const RasterLate<const SceneCfg*, const DrawDev*> rest{
+            svc_ptr<float>(&j->attrs), svc_ptr<float>(&j->uvat),        svc_ptr<DrawDev>(&j->draws),
+            in.scenes,                 svc_ptr_mut<SceneRun>(&j->runs), nullptr};
         const auto late = [&] { return rest; };
         raster_tile<false, 4>(late, in, t, 0u, uint4{}, lut, sh, st0, st1, st2, st3, st4);
         pend_e = e;
