@@ -1112,7 +1112,10 @@ int frame_impl(rz_ctx* c, uint32_t* host_out, uint32_t* dev_out, uint32_t* host_
     if (!rc && ring && c->replays) rc = rb.start();  // those pieces came before the replayed job
     release_job(c);
     c->clear_depth = c->next_clear_depth;
-    if (rc) return rc;
+    if (rc) {
+        if (ring) (void)hipStreamSynchronize(c->stream);  // no piece is left on its way into the ring
+        return rc;
+    }
     // on the context's stream (non-blocking), so that a running raster
     // service, whose stream the null stream waits for, does not hold them up
     if (host_out && !ring)
