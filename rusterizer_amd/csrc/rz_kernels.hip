@@ -1488,6 +1488,11 @@ __global__ __launch_bounds__(256) void k_tile_prep(JobBufs b) {
 // eight launches take about 35 us however small the job; the host's rule
 // (direct_binning) draws the line. Tile records are written here too.
 // ---------------------------------------------------------------------------
+// Workgroups of 1024 threads where no CU would hold two of 256 and there are prims
+// enough for them (us, 256 and 1024 threads): 512x512, 256 tiles: 2,000 triangles 5.8
+// and 5.8, 4,000 6.8 and 6.0, 15,000 15.2 and 10.4; 704x704, 484 tiles: 8,000 13.5 and
+// 13.6; 641x479, 315 tiles: 3,001 6.4 and 9.0.
+constexpr uint32_t TILE_BIN_WIDE_TILES = 256, TILE_BIN_WIDE_CHUNKS = 16;
 __device__ __forceinline__ uint32_t find_scene_ftile(const SceneCfg* __restrict__ sc, uint32_t ns, uint32_t t) {
     uint32_t lo = 0, hi = ns;
     while (hi - lo > 1) {
@@ -1498,12 +1503,13 @@ __device__ __forceinline__ uint32_t find_scene_ftile(const SceneCfg* __restrict_
     return lo;
 }
 
-__global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __restrict__ pbin,
+template <uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void k_tile_bin(JobBufs b, const uint4* __restrict__ pbin,
                                                   const SceneCfg* __restrict__ scenes,
                                                   const SceneRun* __restrict__ runs) {
     constexpr uint32_t ROUND = 2048;  // entries written per round
     __shared__ unsigned long long hits[DIRECT_WORDS];
-    __shared__ uint32_t idx[ROUND], scan_lds[4], list_base;
+    __shared__ uint32_t idx[ROUND], scan_lds[THREADS / 64u], list_base;
     if (uniform(b.cnt->overflow) != 0) return;
     const uint32_t nft = uniform(b.head->nftiles), ns = uniform(b.head->nscenes);
     const uint32_t t = threadIdx.x, wave = uniform(t >> 6), lane = t & 63u;
@@ -1511,9 +1517,9 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
     // from k_setup's per-wave counts: few workgroups add to one counter
     constexpr uint32_t ADDERS = 32;
     if (blockIdx.x < ADDERS) {
-        const uint32_t n = b.head->ntri / 64u, step = min(gridDim.x, ADDERS) * 256u;
+        const uint32_t n = b.head->ntri / 64u, step = min(gridDim.x, ADDERS) * THREADS;
         uint32_t pairs = 0, all;
-        for (uint32_t i = blockIdx.x * 256u + t; i < n; i += step) pairs += b.wave_pairs[i];
+        for (uint32_t i = blockIdx.x * THREADS + t; i < n; i += step) pairs += b.wave_pairs[i];
         (void)block_exclusive_scan<uint32_t>(pairs, scan_lds, &all);
         if (t == 0 && all != 0) atomicAdd(&b.cnt->pairs_binned, all);
     }
@@ -1531,14 +1537,14 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
         typedef short Pair __attribute__((ext_vector_type(2)));
         const Pair sign = {-1, 1}, cx = {(short)(ox + 31u), (short)(-1 - (int)ox)},
                    cy = {(short)(oy + 31u), (short)(-1 - (int)oy)};
-        constexpr uint32_t AHEAD = 4;
-        for (uint32_t w0 = wave; w0 < words; w0 += 4u * AHEAD) {
+        constexpr uint32_t AHEAD = 4, WAVES = THREADS / 64u;
+        for (uint32_t w0 = wave; w0 < words; w0 += WAVES * AHEAD) {
             uint4 v[AHEAD];
 #pragma unroll
-            for (uint32_t k = 0; k < AHEAD; ++k) v[k] = pb[min((w0 + 4u * k) * 64u + lane, P - 1u)];
+            for (uint32_t k = 0; k < AHEAD; ++k) v[k] = pb[min((w0 + WAVES * k) * 64u + lane, P - 1u)];
 #pragma unroll
             for (uint32_t k = 0; k < AHEAD; ++k) {
-                const uint32_t w = w0 + 4u * k;
+                const uint32_t w = w0 + WAVES * k;
                 Pair bx, by;
                 __builtin_memcpy(&bx, &v[k].y, 4);
                 __builtin_memcpy(&by, &v[k].z, 4);
@@ -1552,7 +1558,7 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
         }
         __syncthreads();
         // thread t's words, in order: their hits, and the hits before them
-        const uint32_t per = (words + 255u) / 256u, wb = min(t * per, words), we = min(wb + per, words);
+        const uint32_t per = (words + THREADS - 1u) / THREADS, wb = min(t * per, words), we = min(wb + per, words);
         uint32_t own = 0, total;
         for (uint32_t w = wb; w < we; ++w) own += (uint32_t)__popcll(hits[w]);
         const uint32_t before = block_exclusive_scan<uint32_t>(own, scan_lds, &total);
@@ -1576,7 +1582,7 @@ __global__ __launch_bounds__(256) void k_tile_bin(JobBufs b, const uint4* __rest
                         if (pos < ROUND) idx[pos] = w * 64u + (uint32_t)__builtin_ctzll(m);
                 __syncthreads();
                 const uint32_t n = min(total - lo, ROUND);
-                for (uint32_t k = t; k < n; k += 256u) {
+                for (uint32_t k = t; k < n; k += THREADS) {
                     const uint4 e = pb[idx[k]];
                     const uint32_t qm = fine_quad_bits(5u, e.y & 0xFFFFu, e.y >> 16, e.z & 0xFFFFu, e.z >> 16, ox, oy);
                     b.flist[base + lo + k] = make_uint2(runs[s].prim_base + idx[k], zlo_key(e.w, 16u) | qm);
@@ -3048,7 +3054,10 @@ void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_s
                                               b.clip_out);
     if (ev_bin) (void)hipEventRecord(ev_bin, s);
     if (g.direct != 0) {
-        k_tile_bin<<<g.direct, 256, 0, s>>>(b, b.pbin, b.scenes, b.runs);
+        if (g.direct <= TILE_BIN_WIDE_TILES && g.tris >= TILE_BIN_WIDE_CHUNKS)
+            k_tile_bin<1024><<<g.direct, 1024, 0, s>>>(b, b.pbin, b.scenes, b.runs);
+        else
+            k_tile_bin<256><<<g.direct, 256, 0, s>>>(b, b.pbin, b.scenes, b.runs);
     } else {
         k_bin<false><<<at_least1(g.bins), 256, 0, s>>>(b, b.pchunk_scene, b.scenes, b.runs, b.pbin, b.bin_offsets);
         launch_scan<uint32_t>(s, b.bin_counts, b.bin_offsets, b.mat_cap, &b.cnt->mat_len, b.parts,

@@ -60,6 +60,15 @@ def test_tile_bin_equals_two_level_binning(n, width, height, size):
     assert_parity(a, run_oracle(sc), where=sc.name)
 
 
+@pytest.mark.parametrize("n,width,height", [(3840, 512, 512), (3841, 512, 512), (4096, 513, 512), (16384, 33, 31)])
+def test_tile_bin_by_narrow_and_wide_workgroups(n, width, height):
+    """Either side of the rule for 1024 threads (16 chunks of 256, 256 tiles)."""
+    sc = _frame(n, width, height, 6, seed=n + width)
+    print(sc.name, flush=True)
+    for out in (run_gpu(sc, msaa=True), run_batch([sc])[0][0]):
+        assert_parity(out, run_oracle(sc), where=sc.name)
+
+
 def test_tile_bin_batches_switch_between_the_binnings():
     """Batches of small scenes, then with one scene too large, then small
     again, on one context (each binning keeps a graph of its own)."""
