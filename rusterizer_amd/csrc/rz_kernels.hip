@@ -115,6 +115,16 @@ __device__ __forceinline__ void load_vertex(const DrawDev& dd, uint32_t vi, floa
     }
 }
 
+// Whether the job has overflowed and the kernel is to do nothing. `own` are the bits
+// that the kernel raises itself. They are not looked at: they can go up between the
+// loads of two waves of a workgroup, and a workgroup that lost some of its waves
+// would go on with LDS that those never wrote. The others were raised by earlier
+// launches and no longer change, so a workgroup leaves whole or stays whole. (It
+// also makes the total that a replay is sized by the whole job's.)
+__device__ __forceinline__ bool job_stopped(const JobBufs& b, uint32_t own) {
+    return (uniform(b.cnt->overflow) & ~own) != 0u;
+}
+
 // ---------------------------------------------------------------------------
 // Job start: one launch brings the job tables from the host (read over PCIe,
 // where a copy of its own took 4 us before the first kernel), zeroes the
@@ -1510,7 +1520,7 @@ __global__ __launch_bounds__(THREADS) void k_tile_bin(JobBufs b, const uint4* __
     constexpr uint32_t ROUND = 2048;  // entries written per round
     __shared__ unsigned long long hits[DIRECT_WORDS];
     __shared__ uint32_t idx[ROUND], scan_lds[THREADS / 64u], list_base;
-    if (uniform(b.cnt->overflow) != 0) return;
+    if (job_stopped(b, OVF_FINE)) return;
     const uint32_t nft = uniform(b.head->nftiles), ns = uniform(b.head->nscenes);
     const uint32_t t = threadIdx.x, wave = uniform(t >> 6), lane = t & 63u;
     // the coarse entries the job would have had (a count callers can read),

@@ -1,0 +1,59 @@
+"""Small jobs whose first pass outgrows a buffer: which one it was is in the
+overflow bits, one larger pass follows (what the first one counted is the whole
+job's need), and the images equal the oracle's."""
+import numpy as np
+import pytest
+
+from rusterizer_amd import hostmath as hm
+from rusterizer_amd import scenes
+from tests.harness import assert_parity, run_batch, run_gpu, run_oracle
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+OVF_FINE = 16
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    from tests.conftest import gpu_available
+
+    if not gpu_available():
+        pytest.skip("no GPU")
+
+
+def _column(n, width, height, seed):
+    """n triangles as tall as the screen, at distinct depths: each is on the
+    list of every 32-pixel tile of a narrow, high screen."""
+    rng = np.random.default_rng(seed)
+    x = rng.uniform(-0.9, 0.9, (n, 1))
+    corners = np.array([[0.0, -1.0], [0.1, 1.0], [-0.1, 1.0]])
+    xy = corners[None] + np.stack([x, np.zeros_like(x)], -1)
+    pos = np.concatenate([xy, rng.uniform(-0.9, 0.9, (n, 3, 1))], -1).clip(-1, 1)
+    e1, e2 = pos[:, 1] - pos[:, 0], pos[:, 2] - pos[:, 0]
+    back = e1[:, 0] * e2[:, 1] - e1[:, 1] * e2[:, 0] > 0
+    pos[back] = pos[back][:, [0, 2, 1]]
+    eye = hm.identity()
+    return scenes.Scene(f"column{n}_{width}x{height}", width, height, pos.reshape(-1, 3).astype(F),
+                        rng.random((3 * n, 4)).astype(F), None, np.arange(3 * n, dtype=np.uint32), eye, eye, eye,
+                        scenes.FS_COLOR)
+
+
+def test_lists_of_a_batch_outgrow_their_first_estimate():
+    """Eight scenes of 128 tiles and 256 triangles: 262,144 entries, where a
+    new context has room for 174,080."""
+    batch = [_column(256, 2, 4096, seed=s) for s in range(8)]
+    out, stats = run_batch(batch)
+    print(stats, flush=True)
+    assert stats["replays"] == 1 and stats["overflow_bits"] == OVF_FINE
+    for sc, g in zip(batch, out):
+        assert_parity(g, run_oracle(sc), where=sc.name)
+
+
+def test_lists_of_one_scene_outgrow_their_first_estimate():
+    """512 tiles and 5,600 triangles: 2.87 million entries, neither placed side by
+    side nor within the 2.62 million that a new context has room for."""
+    sc = _column(5600, 3, 16384, seed=9)
+    g = run_gpu(sc)
+    print(g["stats"], flush=True)
+    assert g["stats"]["replays"] == 1 and g["stats"]["overflow_bits"] == OVF_FINE
+    assert_parity(g, run_oracle(sc), where=sc.name)
