@@ -947,10 +947,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     __shared__ uint32_t poff[256], pcls[256];  // per triangle of the chunk: first prim (chunk-relative), class
     __shared__ uint32_t wtot[4];               // per wave of the chunk: its prims
     __shared__ uint32_t woff[256];             // one scene: prims before each wave's triangles
-    if (uniform(b.cnt->overflow) != 0) return;
+    const bool one = b.one_scene != 0;
+    if (job_stopped(b, one ? OVF_PRIMS : 0u)) return;
     const uint32_t NT = b.head->ntri;
     const uint32_t prim_cap = b.prim_cap;
-    const bool one = b.one_scene != 0;
     if (one) {
         // k_scene_prep's work for a single small scene, by every workgroup for
         // itself: 64 chunks of four waves are one count a thread, where the
@@ -959,8 +959,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         const uint32_t before = block_exclusive_scan<uint32_t>(
             threadIdx.x < NT / 64u ? b.wave_prims[threadIdx.x] : 0u, wtot, &total);
         woff[threadIdx.x] = before;
+        const uint32_t nch = (total + CHUNK - 1u) / CHUNK;
+        const bool fits = nch * CHUNK <= prim_cap;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            const uint32_t nch = (total + CHUNK - 1u) / CHUNK;
             SceneRun& r = b.runs[0];
             r.prim_off = 0;
             r.nprims = total;
@@ -971,8 +972,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             b.cnt->nprims_raw = total;
             b.cnt->nchunks = nch;
             b.cnt->nprims = nch * CHUNK;
-            if (nch * CHUNK > prim_cap) atomicOr(&b.cnt->overflow, OVF_PRIMS);
+            if (!fits) atomicOr(&b.cnt->overflow, OVF_PRIMS);
         }
+        if (!fits) return;  // (the same in every thread)
         __syncthreads();
     }
     // the chunk table words of the workgroup's next chunk are loaded one
@@ -1032,7 +1034,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         // one thread per prim of the chunk: an input triangle (class 1) or one
         // fan triangle of a clipped polygon (class 2 + slot), so clipped
         // triangles' fans spread over the workgroup
-        bool ovf = false;
         for (uint32_t pp = threadIdx.x; pp < nblk; pp += 256u) {
             // the chunk's triangle owning prim pp: the last one starting at or before it
             uint32_t j = 0;
@@ -1060,13 +1061,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                     for (int i = 0; i < 6; ++i) tv[q].a[i] = pv[4 + i];
                 }
             }
-            if (prim < prim_cap) {
+            if (prim < prim_cap) {  // (all are, or the job was stopped before)
                 const uint2 bb = setup_prim(tv, W, H, d, fs, tex_idx32, proofs, staged ? stage + pp : b.geom + prim,
                                             b.attrs + (size_t)prim * ATTR_STRIDE, b.uvat + (size_t)prim * UV_STRIDE,
                                             b.pbin + prim);
                 if (per_bin != 0) pairs += bins_covered(bb.x, per_bin) * bins_covered(bb.y, per_bin);
-            } else {
-                ovf = true;
             }
         }
         if (per_bin != 0) {
@@ -1081,7 +1080,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             for (uint32_t i = threadIdx.x; i < n16; i += 256u) dst[i] = src[i];
         }
         __syncthreads();  // the stage and the chunk tables are reused by the next chunk
-        if (__ballot(ovf) && lane_id() == 0) atomicOr(&b.cnt->overflow, OVF_PRIMS);
     }
 }
 

@@ -10,7 +10,7 @@ from tests.harness import assert_parity, run_batch, run_gpu, run_oracle
 
 pytestmark = pytest.mark.gpu
 F = np.float32
-OVF_FINE = 16
+OVF_PRIMS, OVF_FINE = 1, 16
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -56,4 +56,15 @@ def test_lists_of_one_scene_outgrow_their_first_estimate():
     g = run_gpu(sc)
     print(g["stats"], flush=True)
     assert g["stats"]["replays"] == 1 and g["stats"]["overflow_bits"] == OVF_FINE
+    assert_parity(g, run_oracle(sc), where=sc.name)
+
+
+def test_prims_of_one_scene_outgrow_their_first_estimate():
+    """1,400 triangles that clipping makes 9,559 of, where a new context has room
+    for 7,840."""
+    sc = scenes.nine_vertex_scene(1400)
+    g = run_gpu(sc)
+    print(g["stats"], flush=True)
+    assert g["stats"]["prims"] == 9559
+    assert g["stats"]["replays"] == 1 and g["stats"]["overflow_bits"] == OVF_PRIMS
     assert_parity(g, run_oracle(sc), where=sc.name)
