@@ -1145,7 +1145,7 @@ __global__ __launch_bounds__(256) void k_bin(JobBufs b, const uint32_t* __restri
     __shared__ uint32_t wbase[SCATTER ? BIN_WORDS * MAX_BINS : 1];
     __shared__ uint32_t wpre[CHUNK];  // first wide (prim, bin) pair of each slot
     __shared__ uint32_t scan_lds[CHUNK / 64];
-    if (uniform(b.cnt->overflow) != 0) return;
+    if (job_stopped(b, SCATTER ? OVF_PAIRS : 0u)) return;
     const uint32_t NC = uniform(b.cnt->nchunks);
     const uint32_t t = threadIdx.x, w = t >> 5, below = (1u << (t & 31)) - 1u;
     bool ovf = false;
@@ -1362,7 +1362,7 @@ __global__ __launch_bounds__(256) void k_fine_bin(JobBufs b, const uint2* __rest
     // the bin's local tiles in place of the scene's bins
     __shared__ uint32_t bits[BIN_WORDS * MAX_BINS];
     __shared__ uint32_t wbase[SCATTER ? BIN_WORDS * MAX_BINS : 1];
-    if (uniform(b.cnt->overflow) != 0) return;
+    if (job_stopped(b, OVF_FINE)) return;  // (too large a matrix: all leave below)
     const uint32_t NCH = uniform(min(b.cnt->fine_chunks, b.fchunk_cap));
     if (uniform(b.cnt->fmat_len) > b.fmat_cap) {
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&b.cnt->overflow, OVF_FINE);

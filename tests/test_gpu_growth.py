@@ -10,7 +10,7 @@ from tests.harness import assert_parity, run_batch, run_gpu, run_oracle
 
 pytestmark = pytest.mark.gpu
 F = np.float32
-OVF_PRIMS, OVF_FINE = 1, 16
+OVF_PRIMS, OVF_PAIRS, OVF_FINE = 1, 4, 16
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -67,4 +67,15 @@ def test_prims_of_one_scene_outgrow_their_first_estimate():
     print(g["stats"], flush=True)
     assert g["stats"]["prims"] == 9559
     assert g["stats"]["replays"] == 1 and g["stats"]["overflow_bits"] == OVF_PRIMS
+    assert_parity(g, run_oracle(sc), where=sc.name)
+
+
+@pytest.mark.parametrize("n,width,height,bits,tiles", [
+    (17000, 3, 4096, OVF_PAIRS, {}),  # 256 bins of 16x16, room for 64,480 entries
+    (20000, 256, 256, OVF_FINE, dict(coarse_bin=256, fine_tile=16))])  # one bin; room for 592,640 entries
+def test_lists_of_the_two_level_binning_outgrow_their_first_estimate(n, width, height, bits, tiles):
+    sc = _column(n, width, height, seed=n)
+    g = run_gpu(sc, **tiles)
+    print(g["stats"], flush=True)
+    assert g["stats"]["replays"] == 1 and g["stats"]["overflow_bits"] == bits
     assert_parity(g, run_oracle(sc), where=sc.name)

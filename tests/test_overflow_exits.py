@@ -31,7 +31,7 @@ def _bits(expr):
     return set(re.findall(r"OVF_\w+", expr))
 
 
-@pytest.mark.parametrize("name", ["k_setup", "k_tile_bin"])
+@pytest.mark.parametrize("name", ["k_setup", "k_bin", "k_fine_bin", "k_tile_bin"])
 def test_kernel_does_not_leave_on_a_bit_it_raises(name):
     body = KERNELS[name]
     raised = set().union(*map(_bits, re.findall(r"atomicOr\(&b\.cnt->overflow,([^;]*)\)", body)))
