@@ -130,6 +130,7 @@ struct JobPlan {
     uint32_t max_nb = 1, max_T = 1;
     uint64_t tris = 0;  // input triangles
     bool direct = false;   // binned by k_tile_bin
+    bool wide = false;     // with 1024 threads a tile
     uint32_t nftiles = 0;  // 32x32 tiles
 };
 
@@ -207,9 +208,9 @@ struct rz_ctx {
     uint64_t gen = 0;  // bumped whenever a buffer moves (invalidates the graph)
 
     // graphs of the launch sequence: with coarse and fine binning, with
-    // k_tile_bin, and that without k_scene_prep (a context that serves jobs of
-    // several kinds keeps them all)
-    JobGraph graphs[3];
+    // k_tile_bin, and that without k_scene_prep, the last two with either width
+    // of k_tile_bin (a context that serves jobs of several kinds keeps them all)
+    JobGraph graphs[5];
     uint32_t tiles_cap = 0;  // raster grid of the graphs: most tiles of any job so far
 
     // frames read back to pageable host memory pass through a pinned ring
@@ -322,17 +323,29 @@ void scene_bins(uint32_t W, uint32_t H, uint32_t req_cb, uint32_t target, uint32
 // (20.6) 184, 171; 32 scenes of 256-512 px (19) 283, 275.
 constexpr uint64_t DIRECT_WORK = 16ull << 20;
 constexpr uint64_t DIRECT_TILE = 1024;
+// Whether it then takes 1024 threads a tile instead of 256: where no CU has two
+// tiles to work on and some scene has prims enough for 16 waves. Kernel alone, us
+// with 256 and 1024 threads (256 CUs):
+//   one scene, 4,000 triangles: 64 tiles 7.3, 6.1; 256 tiles 6.7, 5.9; 289 tiles 6.9, 9.2
+//   one scene, 2,000: 64 tiles 5.7, 5.8; 256 tiles 5.6, 5.8
+//   256 tiles: 16 scenes of 4,000 11.8, 10.5; of 1,000 9.2, 9.4; 64 of 200 10.0, 10.8
+//   16 scenes of 10: 64 tiles 6.5, 7.0; 256 tiles 6.9, 7.3
+// (15,000 triangles gain beyond that, 484 tiles 17.7, 15.6, and lose from there on,
+// 576 tiles 18.8, 20.1.)
+constexpr uint64_t WIDE_TRIS = 3840;
 
 struct DirectRule {
-    uint64_t work = 0, ftiles = 0;
+    uint64_t work = 0, ftiles = 0, most = 0;
     bool fits = true;
     void scene(uint32_t W, uint32_t H, uint64_t tris) {
         const uint64_t ft = (uint64_t)((W + 31) / 32) * ((H + 31) / 32);
         ftiles += ft;
         work += ft * (tris + DIRECT_TILE);
+        most = std::max(most, tris);
         fits = fits && tris <= DIRECT_TRIS;
     }
     bool direct() const { return fits && work <= DIRECT_WORK && ftiles <= 0xFFFF0000ull; }
+    bool wide(uint32_t n_cu) const { return direct() && most > WIDE_TRIS && ftiles <= n_cu; }
 };
 
 uint32_t clamp_u32(uint64_t v) { return v > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)v; }
@@ -453,6 +466,7 @@ int build_job(rz_ctx* c, JobPlan& pl) {
     // raster order: the scenes' tile ranges densest first (ties in scene
     // order), so that the longest tiles do not trail at the end of the launch
     pl.direct = rule.direct();
+    pl.wide = rule.wide((uint32_t)c->n_cu);
     pl.nftiles = clamp_u32(rule.ftiles);
     if (pl.direct)  // the lists are of 32x32 tiles, whatever side was asked for
         for (uint32_t s = 0; s < ns; ++s) sc[s].fts = 5;
@@ -606,6 +620,7 @@ void plan_sizes(const rz_ctx* c, bool frame, uint32_t nd, uint32_t ns, DrawTris 
         rule.scene(W, H, scene_tris(i));
     }
     pl.direct = rule.direct();
+    pl.wide = rule.wide((uint32_t)c->n_cu);
     pl.nftiles = clamp_u32(rule.ftiles);
     pl.ntri = clamp_u32(tri);
     pl.ntiles = clamp_u32(tiles);
@@ -821,6 +836,7 @@ JobGrid job_grid(const rz_ctx* c, const JobPlan& pl, bool for_graph) {
     g.ntiles = for_graph ? std::max(c->tiles_cap, pl.ntiles) : pl.ntiles;
     // (a graph's: 32x32 tiles are at least a quarter of the 16x16 ones)
     if (pl.direct) g.direct = std::max(1u, std::min<uint32_t>(for_graph ? (g.ntiles + 2) / 3 : pl.nftiles, 8192));
+    g.wide = pl.wide;
     return g;
 }
 
@@ -852,7 +868,7 @@ int enqueue_graph(rz_ctx* c, const JobPlan& pl) {
     const int svc = c->job_svc ? c->svc_entry : -1;
     if (pl.ntiles > c->tiles_cap) c->tiles_cap = std::max<uint32_t>(pl.ntiles, c->tiles_cap + c->tiles_cap / 4);
     const JobGrid g = job_grid(c, pl, true);
-    JobGraph& jg = c->graphs[one_scene(pl) ? 2 : pl.direct ? 1 : 0];
+    JobGraph& jg = c->graphs[pl.direct ? 1 + (one_scene(pl) ? 1 : 0) + (pl.wide ? 2 : 0) : 0];
     if (!jg.exec || jg.gen != c->gen || jg.dcap != c->dcap || jg.scap != c->scap || jg.raster != g.raster ||
         jg.tiles != g.ntiles || jg.stats != c->raster_stats || jg.svc != svc) {
         if (jg.exec) {

@@ -229,6 +229,7 @@ struct JobGrid {
     uint32_t raster;     // persistent raster workgroups; 0 = one one-wave workgroup per quadrant
     uint32_t ntiles;     // tiles the one-per-tile raster grid must cover (>= the job's)
     uint32_t direct;     // k_tile_bin blocks; 0 = coarse and fine binning
+    bool wide;           // k_tile_bin with 1024 threads
 };
 
 // A block of words passed to a kernel by value (kernel arguments hold up to

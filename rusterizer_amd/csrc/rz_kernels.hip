@@ -1494,13 +1494,9 @@ __global__ __launch_bounds__(256) void k_tile_prep(JobBufs b) {
 // order, are the tile's list, whose place it reserves with one atomic. The work
 // grows as tiles times prims, all of it 16-byte reads that stay in L2, where the
 // eight launches take about 35 us however small the job; the host's rule
-// (direct_binning) draws the line. Tile records are written here too.
+// (DirectRule) draws the line, and the one between 256 and 1024 threads a tile.
+// Tile records are written here too.
 // ---------------------------------------------------------------------------
-// Workgroups of 1024 threads where no CU would hold two of 256 and there are prims
-// enough for them (us, 256 and 1024 threads): 512x512, 256 tiles: 2,000 triangles 5.8
-// and 5.8, 4,000 6.8 and 6.0, 15,000 15.2 and 10.4; 704x704, 484 tiles: 8,000 13.5 and
-// 13.6; 641x479, 315 tiles: 3,001 6.4 and 9.0.
-constexpr uint32_t TILE_BIN_WIDE_TILES = 256, TILE_BIN_WIDE_CHUNKS = 16;
 __device__ __forceinline__ uint32_t find_scene_ftile(const SceneCfg* __restrict__ sc, uint32_t ns, uint32_t t) {
     uint32_t lo = 0, hi = ns;
     while (hi - lo > 1) {
@@ -3062,7 +3058,7 @@ void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_s
                                               b.clip_out);
     if (ev_bin) (void)hipEventRecord(ev_bin, s);
     if (g.direct != 0) {
-        if (g.direct <= TILE_BIN_WIDE_TILES && g.tris >= TILE_BIN_WIDE_CHUNKS)
+        if (g.wide)
             k_tile_bin<1024><<<g.direct, 1024, 0, s>>>(b, b.pbin, b.scenes, b.runs);
         else
             k_tile_bin<256><<<g.direct, 256, 0, s>>>(b, b.pbin, b.scenes, b.runs);
