@@ -2587,6 +2587,13 @@ __device__ __forceinline__ void report_job(const JobBufs& b) {
     for (uint32_t s = threadIdx.x; s < ns; s += blockDim.x) b.host_flags[s] = b.runs[s].flags;
 }
 
+// The raster kernels' arguments after the JobBufs, in one list for the kernels and
+// for RasterArgs, which k_raster_q reads its own through.
+#define RZ_RASTER_ARGS(ARG)                                                                                        \
+    ARG(PrimGeom, geom) ARG(float, attrs) ARG(float, uvat) ARG(uint2, flist) ARG(uint4, tile_rec)                   \
+    ARG(SceneCfg, scenes) ARG(DrawDev, draws)
+#define RZ_PARAM(T, name) , const T* __restrict__ name
+
 // Persistent raster (raster_per_cu > 0): raster_per_cu workgroups of four
 // waves per CU, each wave one quadrant of the tile its workgroup holds;
 // contiguous bands of tiles become 8 queues, drained XCD-local first. Held
@@ -2594,9 +2601,7 @@ __device__ __forceinline__ void report_job(const JobBufs& b) {
 // faster than unconstrained (6 waves).
 template <bool STATS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8, 8))) void k_raster(
-    JobBufs b, const PrimGeom* __restrict__ geom, const float* __restrict__ attrs, const float* __restrict__ uvat,
-    const uint2* __restrict__ flist,
-    const uint4* __restrict__ tile_rec, const SceneCfg* __restrict__ scenes, const DrawDev* __restrict__ draws) {
+    JobBufs b RZ_RASTER_ARGS(RZ_PARAM)) {
     const RasterIn in{geom, flist, tile_rec, scenes};
     const auto late = [&] { return JobLate{attrs, uvat, (DrawTable)draws, (SceneTable)scenes, b.runs, b.host_oob}; };
     __shared__ float lut[256];
@@ -2678,19 +2683,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STATS ? 1 :
 // there after the walk, so that no scalar registers hold it meanwhile.
 struct RasterArgs {
     JobBufs b;
-    const PrimGeom* geom;
-    const float* attrs;
-    const float* uvat;
-    const uint2* flist;
-    const uint4* tile_rec;
-    const SceneCfg* scenes;
-    const DrawDev* draws;
+#define RZ_FIELD(T, name) const T* name;
+    RZ_RASTER_ARGS(RZ_FIELD)
+#undef RZ_FIELD
 };
 template <bool STATS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(STATS ? 1 : 8, 8))) void k_raster_q(
-    JobBufs b, const PrimGeom* __restrict__ geom, const float* __restrict__ attrs, const float* __restrict__ uvat,
-    const uint2* __restrict__ flist,
-    const uint4* __restrict__ tile_rec, const SceneCfg* __restrict__ scenes, const DrawDev* __restrict__ draws) {
+    JobBufs b RZ_RASTER_ARGS(RZ_PARAM)) {
     const RasterIn in{geom, flist, tile_rec, scenes};
     const auto late = [] {
         typedef const __attribute__((address_space(4))) RasterArgs* Args;
@@ -3092,11 +3091,12 @@ void launch_job(hipStream_t s, const JobBufs& b, const JobGrid& g, bool raster_s
     // workgroup per quadrant
     const bool persistent = g.raster != 0 || b.prim_cap >= PACKED_PRIMS;
     const uint32_t rgrid = g.raster ? g.raster : (persistent ? RASTER_GRID_WIDE : raster_grid_q(g.ntiles));
-#define RZ_RASTER(ST)                                                                                              \
-    if (persistent)                                                                                                  \
-        k_raster<ST><<<rgrid, 256, 0, s>>>(b, b.geom, b.attrs, b.uvat, b.flist, b.tile_rec, b.scenes, b.draws);    \
-    else                                                                                                           \
-        k_raster_q<ST><<<rgrid, 64, 0, s>>>(b, b.geom, b.attrs, b.uvat, b.flist, b.tile_rec, b.scenes, b.draws)
+#define RZ_GIVE(T, name) , b.name
+#define RZ_RASTER(ST)                                                          \
+    if (persistent)                                                            \
+        k_raster<ST><<<rgrid, 256, 0, s>>>(b RZ_RASTER_ARGS(RZ_GIVE));         \
+    else                                                                       \
+        k_raster_q<ST><<<rgrid, 64, 0, s>>>(b RZ_RASTER_ARGS(RZ_GIVE))
     if (raster_stats) {
         RZ_RASTER(true);
         k_rstat_reduce<<<64, 256, 0, s>>>(b, rgrid);
