@@ -1170,9 +1170,12 @@ int mesh_create(rz_ctx* c, const float* pos, const float* color, const float* uv
         // host data: on the context's stream (not held up by a running
         // raster service); device data: on the null stream, ordered after
         // the caller's work there that produced it
-        e = kind == hipMemcpyHostToDevice ? hipMemcpyAsync(*dst, src, bytes, kind, c->stream)
-                                          : hipMemcpy(*dst, src, bytes, kind);
-        if (e == hipSuccess && kind == hipMemcpyHostToDevice) e = hipStreamSynchronize(c->stream);
+        const hipStream_t s = kind == hipMemcpyHostToDevice ? c->stream : nullptr;
+        e = hipMemcpyAsync(*dst, src, bytes, kind, s);
+        // (a copy on the device does not make the host wait by itself, and the
+        // context's stream, which reads the mesh from here on, does not wait for
+        // the null stream)
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return fail(c, RZ_ERR_HIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
         return RZ_OK;
     };
@@ -1185,8 +1188,8 @@ int mesh_create(rz_ctx* c, const float* pos, const float* color, const float* uv
         uint32_t* dmax = nullptr;
         uint32_t hmax = 0;
         hipError_t e = hipMalloc(&dmax, sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMemset(dmax, 0, sizeof(uint32_t));
         if (e == hipSuccess) {
+            launch_fill_u32(c->stream, dmax, 1, 0u);
             launch_max_index(c->stream, m->idx, ni, dmax);
             e = hipMemcpyAsync(&hmax, dmax, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
         }
