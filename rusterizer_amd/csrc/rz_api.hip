@@ -350,7 +350,8 @@ struct DirectRule {
 
 uint32_t clamp_u32(uint64_t v) { return v > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)v; }
 
-// table block layout at capacities (dcap draws, scap scenes)
+// table block layout at capacities (dcap draws, scap scenes), the same in host
+// and device memory (the device's has no matrices: k_job_init multiplies them)
 int ensure_tables(rz_ctx* c, uint32_t nd, uint32_t ns) {
     if (nd <= c->dcap && ns <= c->scap && c->h_job) return RZ_OK;
     uint32_t dcap = std::max<uint32_t>(c->dcap, 16), scap = std::max<uint32_t>(c->scap, 4);
@@ -671,7 +672,6 @@ JobBufs job_bufs(const rz_ctx* c) {
     JobBufs b{};
     b.head = reinterpret_cast<const JobHead*>(c->d_job);
     b.draws = reinterpret_cast<DrawDev*>(c->d_job + c->off_draws);
-    b.mats = reinterpret_cast<const Mat3*>(c->d_job + c->off_mats);
     b.scenes = reinterpret_cast<const SceneCfg*>(c->d_job + c->off_scenes);
     b.runs = c->d_runs;
     b.cnt = c->d_cnt;
@@ -1353,14 +1353,13 @@ bool noalloc_layout(unsigned char* base, uint32_t ntri_pad, const SceneCfg& sc, 
     b = JobBufs{};
     b.head = reinterpret_cast<const JobHead*>(table);
     b.draws = reinterpret_cast<DrawDev*>(table + NA_OFF_DRAW);
-    b.mats = reinterpret_cast<const Mat3*>(table + NA_OFF_MAT);
     b.scenes = reinterpret_cast<const SceneCfg*>(table + NA_OFF_SCENE);
     // the counters and the scene's run side by side: one copy reads both back
     b.cnt = reinterpret_cast<FrameCounters*>(cv.take<NoallocResult>(1));
     b.runs = reinterpret_cast<SceneRun*>(reinterpret_cast<uintptr_t>(b.cnt) + offsetof(NoallocResult, run));
     b.src_head = b.head;
     b.src_draws = b.draws;
-    b.src_mats = b.mats;
+    b.src_mats = reinterpret_cast<const Mat3*>(table + NA_OFF_MAT);
     b.src_scenes = b.scenes;
     b.src_dcap = 1;
     b.init_split = 8;

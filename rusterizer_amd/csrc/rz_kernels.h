@@ -36,9 +36,8 @@ constexpr uint32_t NO_TILE = 0xFFFFFFFFu;
 constexpr uint32_t NO_PRIM = 0xFFFFFFFFu;
 constexpr uint32_t MANY_DRAWS = 0xFFFFFFFFu;
 
-// PrimGeom.flags bits: texture coordinates not proven in bounds (see
-// uv_in_bounds); barycentric arguments finite at covered samples (see finite_bary)
-constexpr uint32_t PRIM_UV_CHECK = 8, PRIM_FINITE_BARY = 16;
+// PrimGeom.flags bit: texture coordinates not proven in bounds (see uv_in_bounds)
+constexpr uint32_t PRIM_UV_CHECK = 8;
 
 // overflow bits: the job must be replayed with larger buffers
 // (OVF_INDEX: not a buffer -- an index is out of range; nothing is rendered)
@@ -154,7 +153,6 @@ static_assert(sizeof(PrimGeom) == 112, "PrimGeom layout");
 struct JobBufs {
     const JobHead* head;
     DrawDev* draws;
-    const Mat3* mats;
     const SceneCfg* scenes;
     SceneRun* runs;
     FrameCounters* cnt;

@@ -899,7 +899,6 @@ __device__ __forceinline__ uint2 setup_prim(const ClipV* tv, uint32_t W, uint32_
               (tie_rule(o.nx2, o.ny2) ? 4u : 0u) | (fs << 8) | (draw << 16);
     if (fs == RZ_FS_TEXTURE && !(proofs && tex_idx32 && uv_in_bounds(tv, w))) o.flags |= PRIM_UV_CHECK;
     const bool finite = proofs && finite_bary(o);
-    if (finite) o.flags |= PRIM_FINITE_BARY;
     // Depth of a covered sample is ((b0*z0 + b1*z1) + b2*z2) with clamped
     // b_i in [0, 1] and 1 - 2^-23 <= b0+b1+b2 <= 2; three roundings later it
     // is >= zlo below, so a sample can pass LESS only where zbuf > zlo.
