@@ -79,3 +79,39 @@ def test_lists_of_the_two_level_binning_outgrow_their_first_estimate(n, width, h
     print(g["stats"], flush=True)
     assert g["stats"]["replays"] == 1 and g["stats"]["overflow_bits"] == bits
     assert_parity(g, run_oracle(sc), where=sc.name)
+
+
+@pytest.mark.parametrize("width,height", [(160, 96), (520, 520), (3001, 1003)])
+def test_read_back_of_a_frame_that_outgrows_its_buffers(width, height):
+    """Through the pinned ring (which a context's second frame starts): the pieces
+    queued behind the first pass are copied again after the larger one."""
+    import torch
+
+    from rusterizer_amd.render import Context
+
+    sc = scenes.nine_vertex_scene(1400, width, height)
+    sc.idx = np.ascontiguousarray(sc.idx.reshape(-1, 3)[:, ::-1]).reshape(-1)  # (they face away as they are)
+    print(width, height, flush=True)
+    dev = torch.zeros(width * height, dtype=torch.int32, device="cuda")
+    ctx = Context(width, height)
+    try:
+        ctx.set_uniforms(sc.world, sc.view, sc.proj)
+        m = ctx.mesh(sc.pos, sc.color, sc.uv, sc.idx)
+        one = ctx.mesh(sc.pos[:3], sc.color[:3], None, np.arange(3, dtype=np.uint32))
+        ctx.draw(one, sc.fs)
+        ctx.resolve()
+        ctx.draw(m, sc.fs)
+        host = ctx.resolve()
+        stats = ctx.frame_stats()
+        assert stats["replays"] >= 1 and stats["overflow_bits"] & OVF_PRIMS, stats
+        ctx.draw(m, sc.fs)
+        ctx.resolve_device(dev.data_ptr())
+        assert ctx.frame_stats()["replays"] == 0
+        assert np.array_equal(host, dev.cpu().numpy().view(np.uint32).reshape(height, width))
+        assert np.unique(host).size > 100
+        if width < 1000:
+            assert np.array_equal(host, run_oracle(sc)["img"])
+        m.destroy()
+        one.destroy()
+    finally:
+        ctx.close()
