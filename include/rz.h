@@ -70,9 +70,9 @@ int rz_create(uint32_t width, uint32_t height, rz_ctx **out);
  *   RZ_CLIP_WIDE=1     clip each polygon with a full 64-lane wave instead of
  *                      8 lanes (same results; exercises the wide clipper)
  *   RZ_EXACT_PATHS=1   use none of the per-triangle proofs that select the
- *                      raster's fast paths (finite barycentric clamps, texel
- *                      reads without bounds checks): same results, slower;
- *                      exercises the exact paths */
+ *                      raster's fast paths (edges and depths by matrix
+ *                      instructions, texel reads without bounds checks): same
+ *                      results, slower; exercises the exact paths */
 /* A further context on the same device sharing ctx's meshes and textures
  * (no reference counterpart: lets several jobs -- frames or batches -- be in
  * flight at once on their own streams over the same resident data). The
@@ -161,8 +161,9 @@ int rz_frame_stats(const rz_ctx *ctx, uint64_t out[11]);
  * with its own size, clear depth and draws; a scene's draws are rendered in
  * the order they were recorded, exactly as rz_draw/rz_resolve would render
  * them in a context of that size, so every scene's output is identical to
- * rendering it alone. The batch runs as one launch sequence (captured once
- * as a HIP graph and replayed while the buffers fit). */
+ * rendering it alone. The batch runs as one launch sequence (launched
+ * directly, or captured once as a HIP graph and replayed while the buffers
+ * fit: see rz_batch_tuning). */
 
 /* Start recording a batch (no frame may be pending, no batch in flight). */
 int rz_batch_begin(rz_ctx *ctx);
@@ -207,11 +208,12 @@ int rz_batch_scene_flags(const rz_ctx *ctx, uint32_t scene, uint32_t *flags);
 /* Batch tuning: bin_target = most coarse bins per scene when choosing the
  * bin side automatically (1..256); raster_per_cu = persistent raster
  * workgroups per CU (0: one single-wave workgroup per 8x8 quadrant);
- * use_graph = replay a captured HIP graph where that is the faster (1:
- * batches with a scene of more than 16384 triangles or of great extent, and
- * frames of at most 65536 triangles that are read back to the host; while
- * profiling is on, frames launch directly) or always launch the kernels
- * directly (0). Between jobs. */
+ * use_graph = replay a captured HIP graph where that is the faster (1) or
+ * always launch the kernels directly (0). With 1, frames replay it if they
+ * are read back to the host and have at most 65536 triangles (and profiling
+ * is off), batches unless they are small. A job is small if none of its
+ * scenes has more than 16384 triangles, and the sum over its scenes of
+ * (32x32 tiles) * (triangles + 1024) is at most 2^24. Between jobs. */
 int rz_batch_tuning(rz_ctx *ctx, uint32_t bin_target, uint32_t raster_per_cu, int use_graph);
 /* The current tuning: [bin_target, raster_per_cu, use_graph]. */
 int rz_batch_get_tuning(const rz_ctx *ctx, uint32_t out[3]);
@@ -249,7 +251,7 @@ int rz_batch_get_tuning(const rz_ctx *ctx, uint32_t out[3]);
  * streams while it runs; the library's own copies from host memory and
  * to host memory use the context's (non-blocking) stream, while
  * rz_mesh_create_device copies on the null stream, after the caller's work
- * there. */
+ * there, and waits for it. */
 int rz_service_start(rz_ctx *ctx, uint32_t wg_per_cu, uint32_t idle_us);
 int rz_service_stop(rz_ctx *ctx);
 int rz_service_attach(rz_ctx *ctx, int on);
@@ -307,8 +309,10 @@ int rz_memory(const rz_ctx *ctx, uint64_t out[3]);
  * a server size a batch to its memory budget before it records it. */
 int rz_batch_need(const rz_ctx *ctx, const rz_batch_item *items, uint32_t n, uint64_t *bytes);
 /* Frees ctx's pipeline buffers (they grow again with the next job, which
- * then re-captures its graph): lets a server give memory back under
- * pressure. Between jobs; meshes, textures and tables stay. */
+ * then re-captures its graph) and the pinned host memory (at most 16 MB, not
+ * in rz_memory's counts) that its frames are read back through: lets a
+ * server give memory back under pressure. Between jobs; meshes, textures and
+ * tables stay. */
 int rz_trim(rz_ctx *ctx);
 /* Side in pixels (8, 16 or 32; 0 = 32) of the screen tiles whose primitive
  * lists binning builds and the raster walks (no reference counterpart: the
@@ -317,7 +321,8 @@ int rz_trim(rz_ctx *ctx);
  * 8x8 quadrant: with 8 each wave walks its own quadrant's list, with 32 four
  * raster tiles share one list. A scene whose coarse bins cannot hold tiles of
  * that side (more than 256 tiles per bin, or a side that does not divide the
- * bin) uses 16. Results do not depend on it. Between jobs; frames and
+ * bin) uses 16; small jobs (see rz_batch_tuning) have no coarse bins and
+ * always use 32. Results do not depend on it. Between jobs; frames and
  * batches. */
 int rz_set_fine_tile(rz_ctx *ctx, uint32_t side);
 /* The side last set (32 by default). */

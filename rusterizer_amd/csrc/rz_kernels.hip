@@ -1942,10 +1942,11 @@ static_assert(offsetof(PrimGeom, nx0) == 24 && offsetof(PrimGeom, pzx) == 48 && 
 // here against about 120 by the reference's steps; 2 to 13% of the prims take
 // those, and look up an exact stored depth only for samples where it decides.
 // Raster of 256 textured scenes 6.55 -> 4.79 ms, of a 1M-triangle 1080p soup
-// 0.419 -> 0.331 ms, of a 4M-triangle 4K terrain 0.348 -> 0.210 ms. (Every
-// stored depth made exact for each such prim, and the records loaded again for
-// the rows: the batch's 5.21 ms where this form took 5.00.) Groups of 8 prims
-// against 4: the terrain's 0.217 against 0.234 ms, the batch the same.
+// 0.419 -> 0.331 ms, of two 4M-triangle 4K terrains, 0.77 million of the triangles
+// left after clipping 0.348 -> 0.210 ms, 1.29 million 0.568 -> 0.316 ms (traced).
+// (Every stored depth made exact for each such prim, and the records loaded again
+// for the rows: the batch's 5.21 ms where this form took 5.00.) Groups of 8 prims
+// against 4: the first terrain's 0.217 against 0.234 ms, the batch the same.
 typedef float MfmaAcc __attribute__((ext_vector_type(16)));
 typedef __bf16 MfmaIn __attribute__((ext_vector_type(8)));
 // prims whose rows are prepared together: 8 lanes each, so 8 fill a wave; four-wave
